@@ -17,7 +17,7 @@
 #include <string>
 #include <vector>
 
-#include "dd_body.h"
+#include "slice.h"
 
 namespace xr {
 
@@ -360,11 +360,48 @@ struct xr_batch3d {
     std::vector<const xr::Plan3d *> plans;
     std::vector<xr::BatchDesc> desc;
     xr::BatchDesc *d_desc = nullptr;
+    // 2D plans (slice.h) instead: their arguments, and the table offsets in the workspace
+    bool slice = false;
+    std::vector<xr::SliceArgs> slices;
+    std::vector<size_t> off_cell, off_vox;
+    xr::SliceArgs *d_slices = nullptr;
     int device = 0;
     size_t ws_cell = 0, ws_vox = 0;
 };
 
 using xr::fail;
+
+namespace {
+
+// One pass of a batch of 2D plans: a launch per (items per thread, waves) in use.
+int run_slice_pass(const xr_batch3d &b, xr::SlicePass pass, const xr::Route &rt, const xr::IOPtrs &io, char *ws,
+                   hipStream_t s)
+{
+    const int n = (int)b.slices.size();
+    xr::SliceLaunch l{};
+    for (int i = 0; i < n; ++i) {
+        l.in[i] = io.in[i];
+        l.out[i] = io.out[i];
+        l.t0[i] = reinterpret_cast<float *>(ws + (rt.cell ? b.off_cell[i] : b.off_vox[i]));
+        l.t1[i] = xr::slice_second_table(*b.plans[i], l.t0[i], b.slices[i].nb);
+    }
+    for (int bg = 1; bg <= 4; bg *= 2)
+        for (int waves = 4; waves <= 16; waves *= 4) {
+            int64_t total = 0;
+            for (int i = 0; i < n; ++i) {
+                const xr::SliceArgs &a = b.slices[i];
+                l.start[i] = (int)total;
+                if (a.bg == bg && a.waves == waves) total += xr::slice_blocks(pass, a);
+                if (total >= INT32_MAX) return fail(XR_EINVAL, "batch too large for one launch");
+            }
+            l.start[n] = (int)total;
+            if (total > 0)
+                xr::slice_run_many(pass, b.plans[0]->kind, rt.kop, bg, waves, b.d_slices, n, l, s);
+        }
+    return XR_OK;
+}
+
+}  // namespace
 
 extern "C" {
 
@@ -377,6 +414,8 @@ int xr_batch3d_create(xr_plan3d *const *plans, int n, const int *num_batch, xr_b
         return fail(XR_EINVAL, "a batch holds 1.." + std::to_string(XR_BATCH_MAX) + " plans");
     std::unique_ptr<xr_batch3d> b(new xr_batch3d());
     size_t off_cell = 0, off_vox = 0;
+    b->slice = true;
+    for (int i = 0; i < n; ++i) b->slice = b->slice && plans[i] && xr::is_slice(plans[i]->p);
     for (int i = 0; i < n; ++i) {
         if (!plans[i]) return fail(XR_EINVAL, "null plan in batch");
         const xr::Plan3d &p = plans[i]->p;
@@ -388,6 +427,15 @@ int xr_batch3d_create(xr_plan3d *const *plans, int n, const int *num_batch, xr_b
             if (p.device != p0.device) return fail(XR_EINVAL, "batched plans must live on one device");
         }
         if (p.nview <= 0) return fail(XR_EINVAL, "batched plans need at least one view");
+        if (b->slice) {
+            b->slices.push_back(xr::make_slice_args(p, num_batch[i]));
+            b->off_cell.push_back(off_cell);
+            b->off_vox.push_back(off_vox);
+            off_cell += xr::slice_table_bytes(p, true, num_batch[i]);
+            off_vox += xr::slice_table_bytes(p, false, num_batch[i]);
+            b->plans.push_back(&p);
+            continue;
+        }
         xr::BatchDesc d{};
         d.hdr = p.d_hdr;
         d.lineC = p.d_lineC;
@@ -420,12 +468,14 @@ int xr_batch3d_create(xr_plan3d *const *plans, int n, const int *num_batch, xr_b
     int prev = -1;
     (void)hipGetDevice(&prev);
     if (prev != b->device) (void)hipSetDevice(b->device);
-    hipError_t e = hipMalloc(&b->d_desc, sizeof(xr::BatchDesc) * n);
-    if (e == hipSuccess)
-        e = hipMemcpy(b->d_desc, b->desc.data(), sizeof(xr::BatchDesc) * n, hipMemcpyHostToDevice);
+    const size_t bytes = b->slice ? sizeof(xr::SliceArgs) * n : sizeof(xr::BatchDesc) * n;
+    void **dst = b->slice ? reinterpret_cast<void **>(&b->d_slices) : reinterpret_cast<void **>(&b->d_desc);
+    const void *src = b->slice ? (const void *)b->slices.data() : (const void *)b->desc.data();
+    hipError_t e = hipMalloc(dst, bytes);
+    if (e == hipSuccess) e = hipMemcpy(*dst, src, bytes, hipMemcpyHostToDevice);
     if (prev >= 0 && prev != b->device) (void)hipSetDevice(prev);
     if (e != hipSuccess) {
-        if (b->d_desc) (void)hipFree(b->d_desc);
+        if (*dst) (void)hipFree(*dst);
         return fail(XR_ENOMEM, std::string("batch descriptor upload failed: ") + hipGetErrorString(e));
     }
     *out = b.release();
@@ -436,6 +486,7 @@ void xr_batch3d_destroy(xr_batch3d *b)
 {
     if (!b) return;
     if (b->d_desc) (void)hipFree(b->d_desc);
+    if (b->d_slices) (void)hipFree(b->d_slices);
     delete b;
 }
 
@@ -452,7 +503,7 @@ int xr_batch3d_execute(const xr_batch3d *b, int op, const float *const *in, floa
 {
     if (!b) return fail(XR_EINVAL, "null batch");
     if (!in || !out) return fail(XR_EINVAL, "null input/output arrays");
-    const int n = (int)b->desc.size();
+    const int n = (int)b->plans.size();
     const xr::Plan3d &p0 = *b->plans[0];
     const xr::Route rt = xr::route(p0, op);
     if (rt.kop < 0) return fail(XR_EINVAL, "unknown operator " + std::to_string(op));
@@ -481,6 +532,16 @@ int xr_batch3d_execute(const xr_batch3d *b, int op, const float *const *in, floa
     if (!xr::valid_rows(R))
         return fail(XR_EINVAL, "tile_rows must be 1, 2, 4, 8 or 16, with at most one of XR_CELL_DIRECT, XR_CELL_LDS");
     if (!xr::valid_chunk(KC)) return fail(XR_EINVAL, "voxel_chunk must be 1, 4, 8, 16, 16 | XR_VOXEL_HALVES or 32 | XR_VOXEL_HALVES");
+    if (b->slice) {
+        hipStream_t s = static_cast<hipStream_t>(stream);
+        char *ws = static_cast<char *>(workspace);
+        int rc = run_slice_pass(*b, rt.cell ? xr::SLICE_IMAGES : xr::SLICE_SINO, rt, io, ws, s);
+        if (!rc) rc = run_slice_pass(*b, rt.cell ? xr::SLICE_CELL : xr::SLICE_VOXEL, rt, io, ws, s);
+        if (rc) return rc;
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return fail(XR_EHIP, std::string("batched launch failed: ") + hipGetErrorString(e));
+        return XR_OK;
+    }
     bool big = false;
     for (const xr::BatchDesc &d : b->desc) big = big || d.big;
     if (big) R = 8;  // tables of 4 GiB and more: the 64-bit general variant with 8-row tiles

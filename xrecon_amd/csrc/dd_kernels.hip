@@ -37,7 +37,7 @@
 #include <algorithm>
 #include <cstdint>
 
-#include "dd_body.h"
+#include "slice.h"
 
 namespace xr {
 
@@ -112,10 +112,17 @@ __global__ __launch_bounds__(kBlock) void k_sino_prefix(const ViewHdr *__restric
 // FUSED (Nv divides kFdkRows, so a row group holds whole views): the workgroup then
 // builds the row-prefix table of its views' columns itself (prefix_column over the
 // filtered samples kept in LDS).  Otherwise it writes the filtered samples to Q[.].y and
-// k_fdk_prefix builds the table.
+// k_fdk_prefix builds the table.  FDK_SLICE (2D): the filtered samples are the 2D gather's
+// table themselves (slice.h).
+//
+// kFdkOut columns per wave give 16 FMAs per LDS read; a 2D slice has so few rows (720
+// views: 12 groups of 64) that kFdkSliceOut columns per wave fill the GPU better (58 us
+// with 16, 48 workgroups).
 constexpr int kFdkRows = kWave;
 constexpr int kFdkOut = 16;
+constexpr int kFdkSliceOut = 4;
 constexpr int kFdkCols = kFdkOut * kWavesPerBlock;
+enum FdkKind : int { FDK_SAMPLES, FDK_FUSED, FDK_SLICE };
 constexpr int kFdkChunk = 64;
 constexpr int kFdkLoads = kFdkRows / kWavesPerBlock;  // samples per thread per chunk
 static_assert(kFdkTapPad >= kFdkCols && kFdkTapPad >= kFdkChunk, "tap table padding must cover the last blocks");
@@ -131,23 +138,24 @@ __global__ __launch_bounds__(kBlock) void k_fdk_taps(const float *__restrict__ h
     }
 }
 
-template <int MODE, int GEO, bool FUSED>
+template <int MODE, int GEO, int KIND, int OUT>
 __global__ __launch_bounds__(kBlock) void k_fdk_filter(const ViewHdr *__restrict__ hdr, const float4 *__restrict__ colt,
                                                        const float *__restrict__ p, const float *__restrict__ wgt,
                                                        const double *__restrict__ T, float2 *__restrict__ Q,
-                                                       SinoArgs a, int64_t nrows)
+                                                       SinoArgs a, int64_t nrows, int bg)
 {
+    constexpr int kOut = OUT, kCols = OUT * kWavesPerBlock;
     __shared__ double tile[kFdkChunk][kFdkRows + 1];  // [sample][row], +1 against bank conflicts
     const int nu = a.nu;
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int64_t g0 = (int64_t)blockIdx.x * kFdkRows;
-    const int ub = blockIdx.y * kFdkCols + wave * kFdkOut;
+    const int ub = blockIdx.y * kCols + wave * kOut;
     // Tb[s - j] is the tap of sample s for output column ub + j: h[s - (ub + j) + nu - 1]
     const double *Tb = T + kFdkTapPad + nu - 1 - ub;
-    double acc[kFdkOut];
+    double acc[kOut];
 #pragma unroll
-    for (int j = 0; j < kFdkOut; ++j) acc[j] = 0.0;
+    for (int j = 0; j < kOut; ++j) acc[j] = 0.0;
     float next[kFdkLoads];  // thread's samples of the next chunk: rows wave + 4 i, column lane
     auto load = [&](int s0) {
         const int s = s0 + lane;
@@ -172,11 +180,11 @@ __global__ __launch_bounds__(kBlock) void k_fdk_filter(const ViewHdr *__restrict
                 const double x = tile[k0 + k][lane];
                 const int t = s0 + k0 + k;
 #pragma unroll
-                for (int j = 0; j < kFdkOut; ++j) acc[j] = fma(x, Tb[t - j], acc[j]);
+                for (int j = 0; j < kOut; ++j) acc[j] = fma(x, Tb[t - j], acc[j]);
             }
         }
     }
-    if (!FUSED) {
+    if (KIND == FDK_SAMPLES) {
         const int64_t g = g0 + lane;
         if (g >= nrows) return;
         const int64_t sv = g / a.nv;
@@ -184,9 +192,24 @@ __global__ __launch_bounds__(kBlock) void k_fdk_filter(const ViewHdr *__restrict
         const bool keep = hdr[sv % a.nview].keep;
         float2 *dst = Q + (sv * (a.nv + 1) + r) * nu;
 #pragma unroll
-        for (int j = 0; j < kFdkOut; ++j) {
+        for (int j = 0; j < kOut; ++j) {
             const int u = ub + j;
             if (u < nu) dst[keep ? u : nu - 1 - u] = make_float2(0.0f, (float)acc[j]);
+        }
+        return;
+    }
+    if constexpr (KIND == FDK_SLICE) {
+        const int64_t row = g0 + lane;
+        if (row >= nrows) return;
+        const int64_t b = row / a.nview;
+        const int v = (int)(row - b * a.nview);
+        const bool keep = hdr[v].keep;
+        float *dst = reinterpret_cast<float *>(Q) + (b / bg * a.nview + v) * (int64_t)(nu + kSlicePad) * bg + b % bg;
+#pragma unroll
+        for (int j = 0; j < kOut; ++j) {
+            const int u = ub + j;
+            if (u < nu) dst[(int64_t)(keep ? u : nu - 1 - u) * bg] = (float)acc[j];
+            else if (u < nu + kSlicePad) dst[(int64_t)u * bg] = 0.0f;
         }
         return;
     }
@@ -483,15 +506,26 @@ void launch_fdk_table(const Plan3d &p, const float *in, const float *weight, con
     const int64_t nrows = (int64_t)nbatch * p.nview * p.geo.nv;
     const dim3 grid((unsigned)ceil_div(nrows, kFdkRows), (unsigned)ceil_div(a.nu, kFdkCols));
     if (kFdkRows % a.nv == 0) {
-        hipLaunchKernelGGL((k_fdk_filter<MODE, GEO, true>), grid, dim3(kBlock), 0, s, p.d_hdr, p.d_col, in, weight, T,
-                           Q, a, nrows);
+        hipLaunchKernelGGL((k_fdk_filter<MODE, GEO, FDK_FUSED, kFdkOut>), grid, dim3(kBlock), 0, s, p.d_hdr, p.d_col, in,
+                           weight, T, Q, a, nrows, 1);
         return;
     }
     // the unfused filter does not depend on the mode or geometry: one instance
-    hipLaunchKernelGGL((k_fdk_filter<SINO_PLAIN, GEO_FLAT, false>), grid, dim3(kBlock), 0, s, p.d_hdr, p.d_col, in,
-                       weight, T, Q, a, nrows);
+    hipLaunchKernelGGL((k_fdk_filter<SINO_PLAIN, GEO_FLAT, FDK_SAMPLES, kFdkOut>), grid, dim3(kBlock), 0, s, p.d_hdr,
+                       p.d_col, in, weight, T, Q, a, nrows, 1);
     hipLaunchKernelGGL((k_fdk_prefix<MODE, GEO>), dim3(ceil_div(a.nu, kBlock), p.nview, nbatch), dim3(kBlock), 0, s,
                        p.d_hdr, p.d_col, Q, a);
+}
+
+// 2D: the filtered samples as the gather's table.
+template <int OUT>
+void launch_fdk_slice(const Plan3d &p, const float *in, const float *weight, const double *T, float2 *Q, int nbatch,
+                      hipStream_t s)
+{
+    const int64_t nrows = (int64_t)nbatch * p.nview;
+    const dim3 grid((unsigned)ceil_div(nrows, kFdkRows), (unsigned)ceil_div(p.geo.nu + kSlicePad, OUT * kWavesPerBlock));
+    hipLaunchKernelGGL((k_fdk_filter<SINO_PLAIN, GEO_FLAT, FDK_SLICE, OUT>), grid, dim3(kBlock), 0, s, p.d_hdr, p.d_col,
+                       in, weight, T, Q, make_sino_args(p, nbatch), nrows, slice_items(nbatch));
 }
 
 }  // namespace
@@ -520,10 +554,21 @@ int execute_fdk(const Plan3d &p, const float *in, float *out, int nbatch, const 
     float2 *Q = static_cast<float2 *>(ws);
     // the taps live where the view-split partial volumes go later (workspace_bytes
     // reserves room for both); the gather runs after the filter stage on the same stream
-    double *T = reinterpret_cast<double *>(static_cast<char *>(ws) + align256(sino_prefix_bytes(p, nbatch)));
+    double *T = reinterpret_cast<double *>(static_cast<char *>(ws) + (is_slice(p) ? slice_table_bytes(p, false, nbatch)
+                                                                                  : align256(sino_prefix_bytes(p, nbatch))));
     const int nu = p.geo.nu;
     hipLaunchKernelGGL(k_fdk_taps, dim3((unsigned)ceil_div(2 * nu - 1 + 2 * kFdkTapPad, kBlock)), dim3(kBlock), 0, s,
                        filter, T, nu);
+    if (is_slice(p)) {
+        const int64_t wide = (int64_t)ceil_div((int64_t)nbatch * p.nview, kFdkRows) * ceil_div(nu, kFdkCols);
+        if (wide >= 1024) launch_fdk_slice<kFdkOut>(p, in, weight, T, Q, nbatch, s);
+        else launch_fdk_slice<kFdkSliceOut>(p, in, weight, T, Q, nbatch, s);
+        const int rc = slice_run(p, SLICE_VOXEL, rt.kop, nullptr, out, nbatch, ws, s);
+        if (rc) return rc;
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return fail(XR_EHIP, std::string("kernel launch failed: ") + hipGetErrorString(e));
+        return XR_OK;
+    }
     const bool at = rt.kop == VOX_AT;
     if (p.kind == GEO_FLAT) at ? launch_fdk_table<SINO_AT, GEO_FLAT>(p, in, weight, T, Q, nbatch, s)
                                : launch_fdk_table<SINO_PLAIN, GEO_FLAT>(p, in, weight, T, Q, nbatch, s);
@@ -549,6 +594,8 @@ size_t workspace_bytes(const Plan3d &p, int op, int nbatch)
     if (nbatch <= 0) return 0;
     const Route rt = route(p, op);
     if (rt.kop < 0) return 0;
+    if (is_slice(p))
+        return slice_table_bytes(p, rt.cell, nbatch) + (op == XR_OP_BACKPROJECTION_W ? align256(fdk_taps_bytes(p)) : 0);
     if (rt.cell) return align256(vol_prefix_bytes(p, nbatch)) * (p.any_y ? 2 : 1);
     size_t tail = split_partial_bytes(p, nbatch);
     if (op == XR_OP_BACKPROJECTION_W) tail = std::max(tail, fdk_taps_bytes(p));  // FDK filter taps
@@ -592,6 +639,16 @@ int execute_phase(const Plan3d &p, int op, int phase, const float *in, float *ou
     const bool stage = cell_mode == XR_CELL_LDS || (cell_mode == 0 && make_cell_args(p, 1).band);
     if (!valid_chunk(voxel_chunk)) return fail(XR_EINVAL, "voxel_chunk must be 1, 4, 8, 16, 16 | XR_VOXEL_HALVES or 32 | XR_VOXEL_HALVES");
 
+    if (is_slice(p)) {
+        // (tile_rows and voxel_chunk have nothing to choose here)
+        int rc = XR_OK;
+        if (do_prefix) rc = slice_run(p, rt.cell ? SLICE_IMAGES : SLICE_SINO, rt.kop, in, nullptr, nbatch, ws, s);
+        if (!rc && do_gather) rc = slice_run(p, rt.cell ? SLICE_CELL : SLICE_VOXEL, rt.kop, nullptr, out, nbatch, ws, s);
+        if (rc) return rc;
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return fail(XR_EHIP, std::string("kernel launch failed: ") + hipGetErrorString(e));
+        return XR_OK;
+    }
     if (rt.cell && cell_blocks(make_cell_args(p, nbatch), 1, p.ncls[0] + p.ncls[1] + p.ncls[2], nbatch) >=
                        ((int64_t)1 << 31))
         return fail(XR_EINVAL, "batch too large for one launch of the cell gather (column groups / 4 x rows x batch "

@@ -11,7 +11,7 @@
 #include <cmath>
 #include <cstring>
 
-#include "dd_body.h"
+#include "slice.h"
 
 namespace xr {
 
@@ -218,6 +218,8 @@ int build_tables(Plan3d &p, const float *angles, PlanTables &t, std::string &err
             t.col[cb0 + c] = float4{(float)d[c], (float)sig[c], (float)(1.0 / (sig[c] * dvv)),
                                     (float)(cone ? d[c + 1] - d[c] : du)};
         t.col[cb0 + nu] = float4{(float)d[nu], 0.0f, 0.0f, 0.0f};
+        if (is_slice(p))
+            for (int c = 0; c < nu + kSlicePad; ++c) t.dcol.push_back((float)d[std::min(c, nu)]);
         h.dlo = (float)d[0];
         h.dhi = (float)d[nu];
         // Span class: the widest column, measured in pixel widths of the line with the

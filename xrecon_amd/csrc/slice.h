@@ -1,0 +1,509 @@
+// 2D operators (one slice seen by one detector row) without prefix tables.
+//
+// The depth overlap of a 2D operator is always 1, so a detector cell is the sum over the
+// lines of (column overlap) x (pixel), and a pixel the sum over the views of (column
+// overlap) x (sample): there is nothing to integrate along z or the rows.  Both gathers
+// read plain copies of their input, reordered so that kSlicePad zeros follow each line
+// (each view's columns) and `bg` batch items lie side by side: one thread computes the
+// overlaps once and applies them to its bg items.  Every item goes through the same
+// operations in the same order whatever bg is, so a batch equals its items' own calls
+// bit for bit, and so does a batch of plans.
+//
+//  * cell gather: a workgroup is one 64-column group of one view; its kSliceSegs waves take
+//    a run of the lines each (kSliceUnroll lines in flight), and their sums are added in
+//    wave order.  One wave walking all lines, as in the 3D gather, left 3 waves per SIMD
+//    waiting on one load per line.
+//  * voxel gather: a workgroup is an 8 x 8 tile of pixels; its waves take the views in
+//    turn, and their sums are added in wave order (no partial volumes in memory).
+//
+// Bound by VALU issue, 60 to 70 % busy (about 20 instructions per line and column, 55 per
+// view and pixel; 3 to 5 and 9 more for each further item), then by the address path.
+// Measured against the prefix-table gathers that served 2D before: 256^2, 720 views, 256
+// columns, one item: projection 124 -> 37 us, FBP's gather 242 -> 100 us; 16 items, 180
+// views, 400 columns: projection 434 -> 120 us, its transpose 1047 -> 130 us.
+#pragma once
+
+#include "dd_body.h"
+
+namespace xr {
+
+constexpr int kSlicePad = 4;     // zeros after each line of the tables
+constexpr int kSliceSegs = 8;    // cell gather: waves per workgroup, each a run of the lines
+constexpr int kSliceUnroll = 4;  // ... and lines in flight per wave
+
+struct SliceArgs {
+    const ViewHdr *hdr;
+    const float4 *lineC, *lineV, *col;
+    const float *dcol;  // Plan3d::d_dcol
+    const CellGroup *cgrp;
+    const int *citems;
+    int nx, ny, nu, nview, maxline, nb;
+    int bg, ng;       // items per thread (1, 2, 4), groups of them
+    int nitems, ncg;  // column groups over all views, per view
+    int any_y, waves; // waves: per workgroup of the voxel gather (4 or 16)
+    float dx, dy, shx, shy, sod, hscale;
+};
+
+// The descriptor flags a one-slice volume seen by a one-row detector.
+inline bool is_slice(const Plan3d &p) { return p.is2d && p.vol.nz == 1 && p.geo.nv == 1; }
+
+// Items per thread.  The overlaps cost as much as four to six items' sums, so a group of 4
+// with an idle place still beats single items from 3 items on.
+inline int slice_items(int nb) { return nb >= 3 ? 4 : nb; }
+
+inline int64_t slice_image_floats(const Plan3d &p, int nb, bool ydrv)
+{
+    const int bg = slice_items(nb), ng = ceil_div(nb, bg);
+    return (int64_t)ng * bg * (ydrv ? (int64_t)p.vol.nx * (p.vol.ny + kSlicePad) : (int64_t)p.vol.ny * (p.vol.nx + kSlicePad));
+}
+inline int64_t slice_sino_floats(const Plan3d &p, int nb)
+{
+    const int bg = slice_items(nb), ng = ceil_div(nb, bg);
+    return (int64_t)ng * bg * p.nview * (p.geo.nu + kSlicePad);
+}
+
+// Waves per workgroup of the voxel gather, from the image alone (a batch sums its views
+// in the same order as its items): 16 where 8 x 8 tiles with 4 waves each would leave the
+// GPU's 8192 resident waves short.
+inline int slice_waves(const Plan3d &p) { return ceil_div(p.vol.nx, 8) * ceil_div(p.vol.ny, 8) >= 4096 ? 4 : 16; }
+
+inline SliceArgs make_slice_args(const Plan3d &p, int nb)
+{
+    SliceArgs a;
+    a.hdr = p.d_hdr; a.lineC = p.d_lineC; a.lineV = p.d_lineV; a.col = p.d_col; a.dcol = p.d_dcol;
+    a.cgrp = p.d_cgrp; a.citems = p.d_citems;
+    a.nx = p.vol.nx; a.ny = p.vol.ny; a.nu = p.geo.nu; a.nview = p.nview; a.maxline = p.maxline; a.nb = nb;
+    a.bg = slice_items(nb); a.ng = ceil_div(nb, a.bg);
+    a.ncg = ceil_div(a.nu, kWave); a.nitems = a.ncg * a.nview;
+    a.any_y = p.any_y; a.waves = slice_waves(p);
+    a.dx = p.vol.dx; a.dy = p.vol.dy; a.shx = p.vol.shift_x; a.shy = p.vol.shift_y; a.sod = p.sod;
+    a.hscale = p.dvv / p.dz;
+    return a;
+}
+
+// Workgroups of the passes.
+__host__ __device__ inline int slice_image_blocks(const SliceArgs &a)
+{
+    return ceil_div(a.nx + kSlicePad, 32) * ceil_div(a.ny + kSlicePad, 32) * a.ng;
+}
+__host__ __device__ inline int64_t slice_cell_blocks(const SliceArgs &a) { return (int64_t)a.nitems * a.ng; }
+__host__ __device__ inline int64_t slice_sino_blocks(const SliceArgs &a)
+{
+    return (int64_t)ceil_div(a.nu + kSlicePad, kBlock) * a.nview * a.ng;
+}
+__host__ __device__ inline int slice_voxel_blocks(const SliceArgs &a)
+{
+    return ceil_div(a.nx, 8) * ceil_div(a.ny, 8) * a.ng;
+}
+
+enum SlicePass : int { SLICE_IMAGES, SLICE_SINO, SLICE_CELL, SLICE_VOXEL };
+
+// One launch over several instances: first block, buffers and tables of each.
+struct SliceLaunch {
+    int start[XR_BATCH_MAX + 1];
+    const float *in[XR_BATCH_MAX];
+    float *out[XR_BATCH_MAX], *t0[XR_BATCH_MAX], *t1[XR_BATCH_MAX];
+};
+
+// slice_kernels.hip
+int64_t slice_blocks(SlicePass pass, const SliceArgs &a);
+// Bytes of the tables the gathers to the sinogram (cell) or to the image read.
+size_t slice_table_bytes(const Plan3d &p, bool cell, int nb);
+float *slice_second_table(const Plan3d &p, void *ws, int nb);
+int slice_run(const Plan3d &p, SlicePass pass, int kop, const float *in, float *out, int nb, void *ws, hipStream_t s);
+void slice_run_many(SlicePass pass, int kind, int kop, int bg, int waves, const SliceArgs *args, int n,
+                    const SliceLaunch &l, hipStream_t s);
+
+#if defined(__HIPCC__)
+
+// N consecutive floats from a 4-byte aligned place, as one load.
+template <int N>
+__device__ inline void slice_load(const char *base, unsigned off, float *dst)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    typedef float vec __attribute__((ext_vector_type(N), aligned(4)));
+    const vec r = *(const __attribute__((address_space(1))) vec *)((const __attribute__((address_space(1))) char *)base + off);
+#pragma unroll
+    for (int i = 0; i < N; ++i) dst[i] = r[i];
+#endif
+}
+
+// 1 / y to within an ulp: v_rcp_f32 and one Newton step (a division compiles to ten
+// instructions).
+__device__ inline float slice_rcp(float y)
+{
+    const float r = __builtin_amdgcn_rcpf(y);
+    return fmaf(fmaf(-y, r, 1.0f), r, r);
+}
+
+// w x, zero where w is zero, whatever x holds: one v_mul_legacy_f32.
+__device__ inline float mul_or_zero(float w, float x)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    float r;
+    asm("v_mul_legacy_f32 %0, %1, %2" : "=v"(r) : "v"(w), "v"(x));
+    return r;
+#else
+    return w == 0.0f ? 0.0f : w * x;
+#endif
+}
+
+// Copies of the images in both line orientations: TX[g][j][m = i][b] and
+// TY[g][i][m = Ny-1-j][b], zeros after each line (32 x 32 tiles, transposed through LDS).
+template <int BG>
+__device__ inline void slice_images(const SliceArgs &a, int bid, const float *__restrict__ f, float *__restrict__ TX,
+                                    float *__restrict__ TY)
+{
+    __shared__ float tile[BG][32][33];
+    const int tx = ceil_div(a.nx + kSlicePad, 32), ty = ceil_div(a.ny + kSlicePad, 32);
+    const int i0 = bid % tx * 32, j0 = bid / tx % ty * 32, g = bid / (tx * ty);
+    const int l = threadIdx.x & 31, r0 = threadIdx.x >> 5;
+    const int64_t plane = (int64_t)a.nx * a.ny;
+    const int px = a.nx + kSlicePad, py = a.ny + kSlicePad;
+#pragma unroll
+    for (int b = 0; b < BG; ++b)
+        for (int r = r0; r < 32; r += 8) {
+            const int i = i0 + l, j = j0 + r;
+            tile[b][r][l] = i < a.nx && j < a.ny && g * BG + b < a.nb ? f[(g * BG + b) * plane + (int64_t)j * a.nx + i] : 0.0f;
+        }
+    __syncthreads();
+    for (int r = r0; r < 32; r += 8) {
+        const int i = i0 + l, j = j0 + r;
+        if (i < px && j < a.ny) {
+            float *d = TX + (((int64_t)g * a.ny + j) * px + i) * BG;
+#pragma unroll
+            for (int b = 0; b < BG; ++b) d[b] = tile[b][r][l];
+        }
+    }
+    if (!a.any_y) return;
+    for (int r = r0; r < 32; r += 8) {
+        const int i = i0 + r, j = j0 + l;
+        if (i < a.nx && j < py) {
+            float *d = TY + (((int64_t)g * a.nx + i) * py + (j < a.ny ? a.ny - 1 - j : j)) * BG;
+#pragma unroll
+            for (int b = 0; b < BG; ++b) d[b] = tile[b][l][r];
+        }
+    }
+}
+
+// Copy of the sinograms, S[g][v][c][b]: columns in internal order, zeros after the last;
+// A^T: times the forward normalisation Delta / (W cos theta) (the height term of the ray
+// is zero in 2D).
+template <bool AT, int GEO, int BG>
+__device__ inline void slice_sino(const SliceArgs &a, int bid, const float *__restrict__ p, float *__restrict__ S)
+{
+    const int gx = ceil_div(a.nu + kSlicePad, kBlock);
+    const int c = bid % gx * kBlock + threadIdx.x, v = bid / gx % a.nview, g = bid / (gx * a.nview);
+    if (c >= a.nu + kSlicePad) return;
+    const ViewHdr h = ro_load(a.hdr + v);
+    float s[BG];
+#pragma unroll
+    for (int b = 0; b < BG; ++b)
+        s[b] = c < a.nu && g * BG + b < a.nb ? p[((int64_t)(g * BG + b) * a.nview + v) * a.nu + (h.keep ? c : a.nu - 1 - c)]
+                                             : 0.0f;
+    if (AT && c < a.nu) {
+        const float4 cc = g_load(a.col + (int64_t)v * (a.nu + 1) + c);
+        float q = h.delta / cc.w;
+        if (GEO != GEO_PAR) {
+            const float dbp = 0.5f * (cc.x + g_load(&a.col[(int64_t)v * (a.nu + 1) + c + 1].x)) - h.P;
+            q /= fabsf(h.S) / sqrtf(dbp * dbp + h.S * h.S);
+        }
+#pragma unroll
+        for (int b = 0; b < BG; ++b) s[b] *= q;
+    }
+    float *d = S + (((int64_t)g * a.nview + v) * (a.nu + kSlicePad) + c) * BG;
+#pragma unroll
+    for (int b = 0; b < BG; ++b) d[b] = s[b];
+}
+
+// FDK weight U of the pixels of one line: at position q along the line, with the terms
+// that do not change on the line (uniform) in u0, u1.
+template <int GEO>
+struct SliceWeight {
+    float u0, u1;
+    __device__ SliceWeight(float sal, float sln, float pln, float sod)
+    {
+        if (GEO == GEO_FLAT) {
+            const float r = 1.0f / (sod * sod);
+            u0 = fmaf(-sln * pln, r, 1.0f);
+            u1 = -sal * r;
+        } else {
+            const float e = sln - pln;
+            u0 = e * e;
+            u1 = sal;
+        }
+    }
+    __device__ float at(float q) const
+    {
+        if (GEO == GEO_PAR) return 1.0f;
+        if (GEO == GEO_FLAT) {
+            const float t = fmaf(q, u1, u0);
+            return slice_rcp(t * t);
+        }
+        const float e = u1 - q;
+        return slice_rcp(fmaf(e, e, u0));
+    }
+};
+
+// Lines L .. L+U-1 of the cell gather: the column's overlap with each of
+// NP consecutive pixels from the first it touches.  A column off the line reads the zeros
+// after it; the third and further pixels count only where they overlap.
+template <int OPK, int GEO, int BG, int NP, int U>
+__device__ inline void slice_lines(const SliceArgs &a, const ViewHdr &h, const float4 *lt, const char *T, int L,
+                                   float d0, float d1, float *acc)
+{
+    const int nal = wave_uniform(h.nalong);
+    const float fal = (float)nal;
+    const unsigned pitch = (unsigned)(nal + kSlicePad) * BG * 4u;
+    float w[U][NP], f[U][NP * BG], lam[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const int Lu = L + u;
+        const float4 lc = ro_load(lt + Lu);
+        const float lo = clampf(fmaf(d0, lc.y, lc.x), 0.0f, fal), hi = clampf(fmaf(d1, lc.y, lc.x), 0.0f, fal);
+        const float mf = floorf(lo);
+        const unsigned m = hi > lo ? (unsigned)lo : (unsigned)nal;
+        lam[u] = lc.w;
+        float e = lo;
+#pragma unroll
+        for (int q = 0; q < NP; ++q) {
+            const float n = q + 1 < NP ? minf_finite(hi, mf + (float)(q + 1)) : hi;
+            w[u][q] = n - e;
+            e = n;
+        }
+        const char *line = T + (int64_t)Lu * pitch;
+        if (BG == 1) {
+            slice_load<NP>(line, m * 4u, f[u]);
+        } else {
+#pragma unroll
+            for (int q = 0; q < NP; ++q) slice_load<BG>(line, m * (BG * 4u) + q * (BG * 4u), f[u] + q * BG);
+        }
+        if (OPK == CELL_BWT) {
+            const float dal = h.xdrv ? a.dx : a.dy, p0 = (0.5f - 0.5f * fal) * dal + (h.xdrv ? a.shx : a.shy);
+            const float pln = h.xdrv ? (0.5f * a.ny - (float)Lu - 0.5f) * a.dy + a.shy
+                                     : ((float)Lu - 0.5f * a.nx + 0.5f) * a.dx + a.shx;
+            const SliceWeight<GEO> U1(h.xdrv ? h.sx : h.sy, h.xdrv ? h.sy : h.sx, pln, a.sod);
+#pragma unroll
+            for (int q = 0; q < NP; ++q) w[u][q] *= U1.at(fmaf(mf + (float)q, dal, p0));
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int b = 0; b < BG; ++b) {
+            float s = w[u][0] * f[u][b];
+#pragma unroll
+            for (int q = 1; q < NP; ++q)
+                s = q < 2 ? fmaf(w[u][q], f[u][q * BG + b], s) : s + mul_or_zero(w[u][q], f[u][q * BG + b]);
+            acc[b] = OPK == CELL_A ? fmaf(lam[u], s, acc[b]) : acc[b] + s;
+        }
+}
+
+// A line on which a column can cover five pixels and more.
+template <int OPK, int GEO, int BG>
+__device__ inline void slice_line_any(const SliceArgs &a, const ViewHdr &h, const float4 &lc, const char *line, int L,
+                                      float d0, float d1, float *acc)
+{
+    const int nal = wave_uniform(h.nalong);
+    const float fal = (float)nal;
+    const float lo = clampf(fmaf(d0, lc.y, lc.x), 0.0f, fal), hi = clampf(fmaf(d1, lc.y, lc.x), 0.0f, fal);
+    const float dal = h.xdrv ? a.dx : a.dy, p0 = (0.5f - 0.5f * fal) * dal + (h.xdrv ? a.shx : a.shy);
+    const float pln = h.xdrv ? (0.5f * a.ny - (float)L - 0.5f) * a.dy + a.shy
+                             : ((float)L - 0.5f * a.nx + 0.5f) * a.dx + a.shx;
+    const SliceWeight<GEO> U1(h.xdrv ? h.sx : h.sy, h.xdrv ? h.sy : h.sx, pln, a.sod);
+    float s[BG];
+#pragma unroll
+    for (int b = 0; b < BG; ++b) s[b] = 0.0f;
+    for (float m = floorf(lo); m < hi; m += 1.0f) {
+        float w = minf_finite(hi, m + 1.0f) - maxf_finite(lo, m);
+        if (OPK == CELL_BWT) w *= U1.at(fmaf(m, dal, p0));
+        float f[BG];
+        slice_load<BG>(line, (unsigned)m * (BG * 4u), f);
+#pragma unroll
+        for (int b = 0; b < BG; ++b) s[b] = fmaf(w, f[b], s[b]);
+    }
+#pragma unroll
+    for (int b = 0; b < BG; ++b) acc[b] = OPK == CELL_A ? fmaf(lc.w, s[b], acc[b]) : acc[b] + s[b];
+}
+
+// Workgroup bid of the cell gather (see the head of the file).
+template <int OPK, int GEO, int BG>
+__device__ inline void slice_cell(const SliceArgs &a, int bid, const float *__restrict__ TX, const float *__restrict__ TY,
+                                  float *__restrict__ out)
+{
+    __shared__ float part[kSliceSegs][BG][kWave];
+    const int lane = threadIdx.x & (kWave - 1), wave = wave_uniform(threadIdx.x / kWave);
+    const int g = bid / a.nitems, item = wave_uniform(ro_load(a.citems + (bid - g * a.nitems)));
+    const int v = item / a.ncg, c = (item - v * a.ncg) * kWave + lane;
+    const ViewHdr h = ro_load(a.hdr + v);
+    const CellGroup cg = ro_load(a.cgrp + item);
+    const float4 *ct = a.col + (int64_t)v * (a.nu + 1) + imin(c, a.nu - 1);
+    const float4 cc = g_load(ct);
+    const float d0 = cc.x, d1 = g_load(&ct[1].x);
+    const float4 *lt = a.lineC + (int64_t)v * a.maxline;
+    const int nline = wave_uniform(h.nline), nal = wave_uniform(h.nalong);
+    const unsigned pitch = (unsigned)(nal + kSlicePad) * BG * 4u;
+    const char *T = reinterpret_cast<const char *>(wave_uniform(h.xdrv) ? TX : TY) + (int64_t)g * nline * pitch;
+    const int per = ceil_div(nline, kSliceSegs), L0 = wave * per, L1 = imin(nline, L0 + per);
+    float acc[BG];
+#pragma unroll
+    for (int b = 0; b < BG; ++b) acc[b] = 0.0f;
+    int L = L0;
+    if (wave_uniform(cg.span) == 2) {
+        for (; L + kSliceUnroll <= L1; L += kSliceUnroll)
+            slice_lines<OPK, GEO, BG, 2, kSliceUnroll>(a, h, lt, T, L, d0, d1, acc);
+        for (; L < L1; ++L) slice_lines<OPK, GEO, BG, 2, 1>(a, h, lt, T, L, d0, d1, acc);
+    } else if (wave_uniform(cg.span) == 3) {
+        for (; L + kSliceUnroll <= L1; L += kSliceUnroll)
+            slice_lines<OPK, GEO, BG, 3, kSliceUnroll>(a, h, lt, T, L, d0, d1, acc);
+        for (; L < L1; ++L) slice_lines<OPK, GEO, BG, 3, 1>(a, h, lt, T, L, d0, d1, acc);
+    } else {
+        // each line on the narrowest path its pixel footprint allows, as in cell_body
+        for (; L < L1; ++L) {
+            const float4 lc = ro_load(lt + L);
+            const float s = cg.wmax * lc.y;
+            if (s < 1.99f) slice_lines<OPK, GEO, BG, 3, 1>(a, h, lt, T, L, d0, d1, acc);
+            else if (s < 2.99f) slice_lines<OPK, GEO, BG, 4, 1>(a, h, lt, T, L, d0, d1, acc);
+            else slice_line_any<OPK, GEO, BG>(a, h, lc, T + (int64_t)L * pitch, L, d0, d1, acc);
+        }
+    }
+#pragma unroll
+    for (int b = 0; b < BG; ++b) part[wave][b][lane] = acc[b];
+    __syncthreads();
+    if (wave >= BG || c >= a.nu || g * BG + wave >= a.nb) return;  // wave b writes item b
+    float s = part[0][wave][lane];
+#pragma unroll
+    for (int k = 1; k < kSliceSegs; ++k) s += part[k][wave][lane];
+    float q = h.colw;
+    if (OPK == CELL_A) {
+        q = h.delta * cc.z / cc.w;  // as cell_store, hb = 0
+        if (GEO != GEO_PAR) {
+            const float dbp = 0.5f * (d0 + d1) - h.P;
+            q /= fabsf(h.S) / sqrtf(dbp * dbp + h.S * h.S);
+        }
+    }
+    out[((int64_t)(g * BG + wave) * a.nview + v) * a.nu + (h.keep ? c : a.nu - 1 - c)] = s * q;
+}
+
+// atan(t) for the column seeds, which are corrected against the table: a least-squares odd
+// polynomial for |t| <= 0.6 (within 3e-7 rad; fans of up to 62 degrees), atanf beyond.
+__device__ inline float slice_atan(float t)
+{
+    if (wave_any(fabsf(t) > 0.6f)) return atanf(t);
+    const float q = t * t;
+    float r = fmaf(q, 0.0563796f, -0.1275247f);
+    r = fmaf(q, r, 0.1980930f);
+    r = fmaf(q, r, -0.3332516f);
+    return fmaf(t * q, r, t);
+}
+
+// One view of the voxel gather: the overlaps of the pixel's footprint [a0, a1] with three
+// columns at a time, from the one that the closed-form inverse gives (corrected where it
+// came out past the footprint's start; columns before it have no width).  XD: x-driven.
+template <int OPK, int GEO, int BG, bool XD>
+__device__ inline void slice_view(const SliceArgs &a, const ViewHdr &h, const float4 &lv, const float *dtab,
+                                  const float *stab, float fm, float pal, float pln, float *acc)
+{
+    const char *dt = reinterpret_cast<const char *>(dtab), *st = reinterpret_cast<const char *>(stab);
+    // both ends on the detector: a pixel off it has no width left
+    const float e = fmaf(fm, lv.y, lv.x);
+    const float a0 = clampf(e, h.dlo, h.dhi), a1 = clampf(e + lv.y, h.dlo, h.dhi);
+    const float T = seed_div(fmaf(h.tp1, a0, h.tp0), fmaf(h.tq1, a0, h.tq0));
+    int c = (int)clampf(fmaf(h.tk1, GEO == GEO_ARC ? slice_atan(T) : T, h.tk0), 0.0f, (float)(a.nu - 1));
+    float d[4], s[3 * BG];
+    auto load = [&]() {
+        slice_load<4>(dt, (unsigned)c * 4u, d);
+        if (BG == 1) {
+            slice_load<3>(st, (unsigned)c * 4u, s);
+        } else {
+#pragma unroll
+            for (int q = 0; q < 3; ++q) slice_load<BG>(st, (unsigned)c * (BG * 4u) + q * (BG * 4u), s + q * BG);
+        }
+    };
+    load();
+    while (wave_any(d[0] > a0)) {  // (d_0 <= a0, so c stays above 0 here)
+        if (d[0] > a0) --c;
+        load();
+    }
+    float sum[BG], b0 = a0;
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+        const float b1 = clampf(d[q + 1], a0, a1);
+#pragma unroll
+        for (int b = 0; b < BG; ++b) {
+            const float x = mul_or_zero(b1 - b0, s[q * BG + b]);
+            sum[b] = q == 0 ? x : sum[b] + x;
+        }
+        b0 = b1;
+    }
+    if (wave_any(d[3] < a1)) {  // pixels over more than three columns
+        for (int k = c + 3; k < a.nu && b0 < a1; ++k) {
+            float dn, x[BG];
+            slice_load<1>(dt, (unsigned)(k + 1) * 4u, &dn);
+            slice_load<BG>(st, (unsigned)k * (BG * 4u), x);
+            const float b1 = clampf(dn, a0, a1);
+#pragma unroll
+            for (int b = 0; b < BG; ++b) sum[b] += mul_or_zero(b1 - b0, x[b]);
+            b0 = b1;
+        }
+    }
+    float hB = 1.0f;
+    if (OPK != VOX_AT) {
+        hB = h.colw * a.hscale * lv.w;
+        if (OPK == VOX_BW) {
+            const SliceWeight<GEO> U(XD ? h.sx : h.sy, XD ? h.sy : h.sx, pln, a.sod);
+            hB *= U.at(pal);
+        }
+    }
+#pragma unroll
+    for (int b = 0; b < BG; ++b) acc[b] = OPK == VOX_AT ? acc[b] + sum[b] : fmaf(hB, sum[b], acc[b]);
+}
+
+// Workgroup bid of the voxel gather over NW waves: wave w takes the views w, w + NW, ...
+template <int OPK, int GEO, int BG, int NW>
+__device__ inline void slice_voxel(const SliceArgs &a, int bid, const float *__restrict__ S, float *__restrict__ out)
+{
+    __shared__ float part[NW][BG][kWave];
+    const int lane = threadIdx.x & (kWave - 1), wave = wave_uniform(threadIdx.x / kWave);
+    const int tx = ceil_div(a.nx, 8), ty = ceil_div(a.ny, 8);
+    const int g = bid / (tx * ty), t = bid - g * (tx * ty);
+    const int i = t % tx * 8 + (lane & 7), j = t / tx * 8 + (lane >> 3);
+    const bool on = i < a.nx && j < a.ny;
+    const int ic = imin(i, a.nx - 1), jc = imin(j, a.ny - 1);
+    const float ppx = ((float)ic - 0.5f * a.nx + 0.5f) * a.dx + a.shx;
+    const float ppy = (0.5f * a.ny - (float)jc - 0.5f) * a.dy + a.shy;
+    const float fx = (float)ic, fy = (float)(a.ny - 1 - jc);
+    const int sp = a.nu + kSlicePad;
+    const float *Sg = S + (int64_t)g * a.nview * sp * BG;
+    float acc[BG];
+#pragma unroll
+    for (int b = 0; b < BG; ++b) acc[b] = 0.0f;
+    // the next view's header and line entry are read during this view's gather
+    auto line_of = [&](int v, const ViewHdr &h) {
+        return g_load(a.lineV + (int64_t)v * a.maxline + (wave_uniform(h.xdrv) ? jc : ic));
+    };
+    ViewHdr hn = ro_load(a.hdr + imin(wave, a.nview - 1));
+    float4 ln = line_of(imin(wave, a.nview - 1), hn);
+    for (int v = wave; v < a.nview; v += NW) {
+        const ViewHdr h = hn;
+        const float4 lv = ln;
+        const int vn = imin(v + NW, a.nview - 1);
+        hn = ro_load(a.hdr + vn);
+        ln = line_of(vn, hn);
+        const float *dt = a.dcol + (int64_t)v * sp, *st = Sg + (int64_t)v * sp * BG;
+        if (wave_uniform(h.xdrv)) slice_view<OPK, GEO, BG, true>(a, h, lv, dt, st, fx, ppx, ppy, acc);
+        else slice_view<OPK, GEO, BG, false>(a, h, lv, dt, st, fy, ppy, ppx, acc);
+    }
+#pragma unroll
+    for (int b = 0; b < BG; ++b) part[wave][b][lane] = acc[b];
+    __syncthreads();
+    if (wave >= BG || !on || g * BG + wave >= a.nb) return;
+    float r = part[0][wave][lane];
+#pragma unroll
+    for (int k = 1; k < NW; ++k) r += part[k][wave][lane];
+    out[((int64_t)(g * BG + wave) * a.ny + j) * a.nx + i] = r;
+}
+
+#endif
+
+}  // namespace xr

@@ -1,0 +1,168 @@
+// Kernels and launches of the 2D operators (slice.h), for one plan and for batches.
+#include <hip/hip_runtime.h>
+
+#include <cstdint>
+
+#include "slice.h"
+
+namespace xr {
+
+namespace {
+
+// A launch covers one plan (SliceOne) or the instances of a batch that share the kernel's
+// template (SliceMany: instances of other item groups count no blocks).
+struct SliceOne {
+    SliceArgs a;
+    const float *in;
+    float *out, *t0, *t1;
+};
+
+struct SliceMany {
+    const SliceArgs *args;  // device array
+    int n;
+    SliceLaunch l;
+};
+
+struct SliceJob {
+    SliceArgs a;
+    const float *in;
+    float *out, *t0, *t1;
+    int bid;
+};
+
+__device__ inline bool slice_job(const SliceOne &o, SliceJob &j)
+{
+    j.a = o.a; j.in = o.in; j.out = o.out; j.t0 = o.t0; j.t1 = o.t1;
+    j.bid = blockIdx.x;
+    return true;
+}
+__device__ inline bool slice_job(const SliceMany &m, SliceJob &j)
+{
+    int bid = blockIdx.x, i = 0;
+    while (i + 1 < m.n && bid >= m.l.start[i + 1]) ++i;
+    if (bid >= m.l.start[m.n]) return false;
+    j.a = ro_load(m.args + i);
+    j.in = m.l.in[i]; j.out = m.l.out[i]; j.t0 = m.l.t0[i]; j.t1 = m.l.t1[i];
+    j.bid = bid - m.l.start[i];
+    return true;
+}
+
+template <int BG, class SRC>
+__global__ __launch_bounds__(kBlock) void k_slice_images(SRC src)
+{
+    SliceJob j;
+    if (slice_job(src, j)) slice_images<BG>(j.a, j.bid, j.in, j.t0, j.t1);
+}
+template <bool AT, int GEO, int BG, class SRC>
+__global__ __launch_bounds__(kBlock) void k_slice_sino(SRC src)
+{
+    SliceJob j;
+    if (slice_job(src, j)) slice_sino<AT, GEO, BG>(j.a, j.bid, j.in, j.t0);
+}
+template <int OPK, int GEO, int BG, class SRC>
+__global__ __launch_bounds__(kSliceSegs *kWave) void k_slice_cell(SRC src)
+{
+    SliceJob j;
+    if (slice_job(src, j)) slice_cell<OPK, GEO, BG>(j.a, j.bid, j.t0, j.t1, j.out);
+}
+template <int OPK, int GEO, int BG, int NW, class SRC>
+__global__ __launch_bounds__(NW *kWave, 8) void k_slice_voxel(SRC src)
+{
+    SliceJob j;
+    if (slice_job(src, j)) slice_voxel<OPK, GEO, BG, NW>(j.a, j.bid, j.t0, j.out);
+}
+
+template <int OPK, int GEO, int BG, class SRC>
+void launch_voxel_nw(int waves, unsigned grid, const SRC &src, hipStream_t s)
+{
+    if (waves == 16) hipLaunchKernelGGL((k_slice_voxel<OPK, GEO, BG, 16, SRC>), dim3(grid), dim3(16 * kWave), 0, s, src);
+    else hipLaunchKernelGGL((k_slice_voxel<OPK, GEO, BG, 4, SRC>), dim3(grid), dim3(4 * kWave), 0, s, src);
+}
+
+template <int GEO, int BG, class SRC>
+void launch_pass(SlicePass pass, int kop, int waves, unsigned grid, const SRC &src, hipStream_t s)
+{
+    const dim3 g(grid), b(kBlock);
+    switch (pass) {
+    case SLICE_IMAGES: hipLaunchKernelGGL((k_slice_images<BG, SRC>), g, b, 0, s, src); break;
+    case SLICE_SINO:
+        if (kop == VOX_AT) hipLaunchKernelGGL((k_slice_sino<true, GEO, BG, SRC>), g, b, 0, s, src);
+        else hipLaunchKernelGGL((k_slice_sino<false, GEO_PAR, BG, SRC>), g, b, 0, s, src);
+        break;
+    case SLICE_CELL:
+        if (kop == CELL_A) hipLaunchKernelGGL((k_slice_cell<CELL_A, GEO, BG, SRC>), g, dim3(kSliceSegs * kWave), 0, s, src);
+        else if (kop == CELL_BT) hipLaunchKernelGGL((k_slice_cell<CELL_BT, GEO_PAR, BG, SRC>), g, dim3(kSliceSegs * kWave), 0, s, src);
+        else hipLaunchKernelGGL((k_slice_cell<CELL_BWT, GEO, BG, SRC>), g, dim3(kSliceSegs * kWave), 0, s, src);
+        break;
+    case SLICE_VOXEL:
+        if (kop == VOX_B) launch_voxel_nw<VOX_B, GEO, BG>(waves, grid, src, s);
+        else if (kop == VOX_BW) launch_voxel_nw<VOX_BW, GEO, BG>(waves, grid, src, s);
+        else launch_voxel_nw<VOX_AT, GEO, BG>(waves, grid, src, s);
+        break;
+    }
+}
+
+template <class SRC>
+void launch_any(SlicePass pass, int kind, int kop, int bg, int waves, unsigned grid, const SRC &src, hipStream_t s)
+{
+#define XR_SLICE_BG(G)                                                          \
+    if (bg == 4) launch_pass<G, 4>(pass, kop, waves, grid, src, s);             \
+    else if (bg == 2) launch_pass<G, 2>(pass, kop, waves, grid, src, s);        \
+    else launch_pass<G, 1>(pass, kop, waves, grid, src, s)
+    if (kind == GEO_FLAT) { XR_SLICE_BG(GEO_FLAT); }
+    else if (kind == GEO_ARC) { XR_SLICE_BG(GEO_ARC); }
+    else { XR_SLICE_BG(GEO_PAR); }
+#undef XR_SLICE_BG
+}
+
+}  // namespace
+
+int64_t slice_blocks(SlicePass pass, const SliceArgs &a)
+{
+    switch (pass) {
+    case SLICE_IMAGES: return slice_image_blocks(a);
+    case SLICE_SINO: return slice_sino_blocks(a);
+    case SLICE_CELL: return slice_cell_blocks(a);
+    case SLICE_VOXEL: return slice_voxel_blocks(a);
+    }
+    return 0;
+}
+
+size_t slice_table_bytes(const Plan3d &p, bool cell, int nb)
+{
+    if (!cell) return align256((size_t)slice_sino_floats(p, nb) * sizeof(float));
+    return align256((size_t)slice_image_floats(p, nb, false) * sizeof(float)) +
+           (p.any_y ? align256((size_t)slice_image_floats(p, nb, true) * sizeof(float)) : 0);
+}
+
+float *slice_second_table(const Plan3d &p, void *ws, int nb)
+{
+    return reinterpret_cast<float *>(static_cast<char *>(ws) +
+                                     align256((size_t)slice_image_floats(p, nb, false) * sizeof(float)));
+}
+
+int slice_run(const Plan3d &p, SlicePass pass, int kop, const float *in, float *out, int nb, void *ws, hipStream_t s)
+{
+    SliceOne o;
+    o.a = make_slice_args(p, nb);
+    o.in = in;
+    o.out = out;
+    o.t0 = static_cast<float *>(ws);
+    o.t1 = slice_second_table(p, ws, nb);
+    const int64_t grid = slice_blocks(pass, o.a);
+    if (grid >= ((int64_t)1 << 31)) return fail(XR_EINVAL, "batch too large for one launch of the 2D gathers");
+    launch_any(pass, p.kind, kop, o.a.bg, o.a.waves, (unsigned)grid, o, s);
+    return XR_OK;
+}
+
+void slice_run_many(SlicePass pass, int kind, int kop, int bg, int waves, const SliceArgs *args, int n,
+                    const SliceLaunch &l, hipStream_t s)
+{
+    SliceMany m;
+    m.args = args;
+    m.n = n;
+    m.l = l;
+    launch_any(pass, kind, kop, bg, waves, (unsigned)l.start[n], m, s);
+}
+
+}  // namespace xr

@@ -109,6 +109,7 @@ struct Plan3d {
     float4 *d_lineC = nullptr;  // [nview][maxline] {toff, invd, iz, lam}: cell kernels
     float4 *d_lineV = nullptr;  // [nview][maxline] {P0, Delta, zeta, 1/(Delta zeta)}: voxel kernels
     float4 *d_col = nullptr;    // [nview][Nu+1]    {d, sigma, kappa, W}
+    float *d_dcol = nullptr;    // 2D: [nview][Nu+4] the column boundaries d alone (d_Nu repeated at the end)
     VoxTile *d_vtile = nullptr; // [nview][ceil(Ny/16)][ceil(Nx/16)]: voxel-gather staging estimates
     CellGroup *d_cgrp = nullptr; // [nview][ceil(Nu/64)]: cell-gather column groups
     int *d_citems = nullptr;     // the groups v * ceil(Nu/64) + g listed by span class (2, then 3, then 0),
@@ -126,6 +127,7 @@ struct Plan3d {
 struct PlanTables {
     std::vector<ViewHdr> hdr;
     std::vector<float4> lineC, lineV, col;
+    std::vector<float> dcol;
     std::vector<VoxTile> vtile;
     std::vector<CellGroup> cgrp;
     std::vector<int> citems;  // as Plan3d::d_citems
