@@ -116,9 +116,9 @@ int xr_plan3d_execute(const xr_plan3d *plan, int op, const float *in, float *out
 #define XR_PHASE_PREFIX 1
 #define XR_PHASE_GATHER 2
 /* voxel_chunk: slices per voxel-gather thread, 1, 4, 8 or 16 (0 = the plan's default);
- * 16 | XR_VOXEL_HALVES runs the 16 slices as two 8-slice halves, 32 | XR_VOXEL_HALVES 32
- * slices as two 16-slice halves, each half skipped by a wave whose lanes have no row of
- * it on the detector (pays on tall volumes). */
+ * 32 | XR_VOXEL_HALVES 32, and 16 | XR_VOXEL_HALVES is 16.  Every form passes over the
+ * groups of 4 slices that have no row on the detector, and all from 4 slices up give the
+ * same results. */
 #define XR_VOXEL_HALVES 0x100
 /* tile_rows: detector rows per cell-gather thread, 1, 2, 4, 8 or 16 (0 = the plan's
  * default).  With 4 rows and more a cell gather may stage, per line, the block of the

@@ -26,6 +26,7 @@ namespace {
 struct BatchDesc {
     const ViewHdr *hdr;
     const float4 *lineC, *lineV, *col;
+    const float *cols;
     const VoxTile *vtile;
     const CellGroup *cgrp;
     const int *citems;  // the plan's column groups by span class (Plan3d::d_citems)
@@ -234,11 +235,11 @@ __global__ __launch_bounds__(kBlock) void k_sino_prefix_batch(const BatchDesc *_
         sino_prefix_body<MODE, GEO>(d.hdr, d.col, io.in[i], reinterpret_cast<float2 *>(ws + d.ws_sino), d.sa, b, v, c);
 }
 
-template <int OPK, int GEO, int KC, bool HALVES>
-__global__ __launch_bounds__(kBlock, KC >= 32 ? 4 : 1) void k_voxel_batch(const BatchDesc *__restrict__ D, int n, BlockStarts st,
+template <int OPK, int GEO, int KC, bool FIT>
+__global__ __launch_bounds__(kBlock, FIT ? (KC >= 32 ? 5 : 6) : KC >= 32 ? 4 : 1) void k_voxel_batch(const BatchDesc *__restrict__ D, int n, BlockStarts st,
                                                         IOPtrs io, char *__restrict__ ws)
 {
-    __shared__ __attribute__((aligned(16))) float2 tile[vox_lds(KC)];
+    __shared__ __attribute__((aligned(16))) float2 tile[FIT ? vox_lds(KC) : vox_lds_rounds(KC, 1)];
     int bid = blockIdx.x;
     const int i = find_instance(st, n, bid);
     if (i < 0) return;
@@ -254,8 +255,8 @@ __global__ __launch_bounds__(kBlock, KC >= 32 ? 4 : 1) void k_voxel_batch(const 
                      : io.out[i];
     int ii, j;
     voxel_coords(bx, by, threadIdx.x, ii, j);
-    voxel_wg<OPK, GEO, KC, HALVES>(d.hdr, d.lineV, d.col, d.vtile, reinterpret_cast<const float2 *>(ws + d.ws_sino),
-                                   dst, a, ii, j, ii < a.nx && j < a.ny, by * gx + bx, (rest % a.nchunk) * KC,
+    voxel_wg<OPK, GEO, KC, 1, FIT>(d.hdr, d.lineV, d.col, d.cols, d.vtile, reinterpret_cast<const float2 *>(ws + d.ws_sino), dst,
+                              a, ii, j, ii < a.nx && j < a.ny, by * gx + bx, (rest % a.nchunk) * KC,
                                    rest / a.nchunk, v0, v1, tile);
 }
 
@@ -313,23 +314,33 @@ void launch_cell_batch(int R, bool big, const BlockStarts *gs, const BatchDesc *
 }
 
 template <int OPK, int GEO>
-void launch_voxel_batch(int KC, const BlockStarts &st, const BatchDesc *D, int n, const IOPtrs &io, char *ws,
+void launch_voxel_batch(int KC, bool fit, const BlockStarts &st, const BatchDesc *D, int n, const IOPtrs &io, char *ws,
                         hipStream_t s)
 {
     const dim3 grid(st.start[n]);
-    switch (KC) {
-    case 1: hipLaunchKernelGGL((k_voxel_batch<OPK, GEO, 1, false>), grid, dim3(kBlock), 0, s, D, n, st, io, ws); break;
-    case 4: hipLaunchKernelGGL((k_voxel_batch<OPK, GEO, 4, false>), grid, dim3(kBlock), 0, s, D, n, st, io, ws); break;
-    case 8: hipLaunchKernelGGL((k_voxel_batch<OPK, GEO, 8, false>), grid, dim3(kBlock), 0, s, D, n, st, io, ws); break;
-    case 16: hipLaunchKernelGGL((k_voxel_batch<OPK, GEO, 16, false>), grid, dim3(kBlock), 0, s, D, n, st, io, ws); break;
-    case 16 | XR_VOXEL_HALVES: hipLaunchKernelGGL((k_voxel_batch<OPK, GEO, 16, true>), grid, dim3(kBlock), 0, s, D, n, st, io, ws); break;
-    default:  // 32 | XR_VOXEL_HALVES: valid_chunk admits nothing else
-        hipLaunchKernelGGL((k_voxel_batch<OPK, GEO, 32, true>), grid, dim3(kBlock), 0, s, D, n, st, io, ws); break;
+#define XR_VOXB(KK, FIT) \
+    hipLaunchKernelGGL((k_voxel_batch<OPK, GEO, KK, FIT>), grid, dim3(kBlock), 0, s, D, n, st, io, ws)
+    switch (chunk_slices(KC)) {
+    case 1: XR_VOXB(1, false); break;
+    case 4: XR_VOXB(4, false); break;
+    case 8:
+        if (fit) XR_VOXB(8, true);
+        else XR_VOXB(8, false);
+        break;
+    case 16:
+        if (fit) XR_VOXB(16, true);
+        else XR_VOXB(16, false);
+        break;
+    default:  // 32: valid_chunk admits nothing else
+        if (fit) XR_VOXB(32, true);
+        else XR_VOXB(32, false);
+        break;
     }
+#undef XR_VOXB
 }
 
 template <int GEO>
-void dispatch_gather(const Route &rt, int R, bool big, int KC, const BlockStarts *gs, const BatchDesc *D, int n,
+void dispatch_gather(const Route &rt, int R, bool big, int KC, bool fit, const BlockStarts *gs, const BatchDesc *D, int n,
                      const IOPtrs &io, char *ws, hipStream_t s)
 {
     if (rt.cell) {
@@ -337,9 +348,9 @@ void dispatch_gather(const Route &rt, int R, bool big, int KC, const BlockStarts
         else if (rt.kop == CELL_BT) launch_cell_batch<CELL_BT, GEO>(R, big, gs, D, n, io, ws, s);
         else launch_cell_batch<CELL_BWT, GEO>(R, big, gs, D, n, io, ws, s);
     } else {
-        if (rt.kop == VOX_B) launch_voxel_batch<VOX_B, GEO>(KC, gs[0], D, n, io, ws, s);
-        else if (rt.kop == VOX_BW) launch_voxel_batch<VOX_BW, GEO>(KC, gs[0], D, n, io, ws, s);
-        else launch_voxel_batch<VOX_AT, GEO>(KC, gs[0], D, n, io, ws, s);
+        if (rt.kop == VOX_B) launch_voxel_batch<VOX_B, GEO>(KC, fit, gs[0], D, n, io, ws, s);
+        else if (rt.kop == VOX_BW) launch_voxel_batch<VOX_BW, GEO>(KC, fit, gs[0], D, n, io, ws, s);
+        else launch_voxel_batch<VOX_AT, GEO>(KC, fit, gs[0], D, n, io, ws, s);
     }
 }
 
@@ -441,6 +452,7 @@ int xr_batch3d_create(xr_plan3d *const *plans, int n, const int *num_batch, xr_b
         d.lineC = p.d_lineC;
         d.lineV = p.d_lineV;
         d.col = p.d_col;
+        d.cols = p.d_cols;
         d.vtile = p.d_vtile;
         d.cgrp = p.d_cgrp;
         d.citems = p.d_citems;
@@ -527,7 +539,12 @@ int xr_batch3d_execute(const xr_batch3d *b, int op, const float *const *in, floa
     }
     if (KC == 0) {
         KC = 1;
-        for (const xr::Plan3d *p : b->plans) KC = std::max(KC, xr::default_chunk(*p));
+        int fit = 31;
+        for (const xr::Plan3d *p : b->plans) {
+            KC = std::max(KC, xr::default_chunk(*p));
+            fit &= p->vox_fit;
+        }
+        while (xr::chunk_slices(KC) > 8 && !(fit & xr::vox_fit_bit(xr::chunk_slices(KC), 1))) KC = xr::chunk_slices(KC) / 2;
     }
     if (!xr::valid_rows(R))
         return fail(XR_EINVAL, "tile_rows must be 1, 2, 4, 8 or 16, with at most one of XR_CELL_DIRECT, XR_CELL_LDS");
@@ -544,6 +561,8 @@ int xr_batch3d_execute(const xr_batch3d *b, int op, const float *const *in, floa
     }
     bool big = false;
     for (const xr::BatchDesc &d : b->desc) big = big || d.big;
+    bool fit = true;  // every block of every instance fits the LDS
+    for (const xr::Plan3d *p : b->plans) fit = fit && (p->vox_fit & xr::vox_fit_bit(xr::chunk_slices(KC), 1));
     if (big) R = 8;  // tables of 4 GiB and more: the 64-bit general variant with 8-row tiles
     hipStream_t s = static_cast<hipStream_t>(stream);
     char *ws = static_cast<char *>(workspace);
@@ -591,9 +610,9 @@ int xr_batch3d_execute(const xr_batch3d *b, int op, const float *const *in, floa
         else if (kind == xr::GEO_ARC) xr::dispatch_sino_prefix<xr::GEO_ARC>(at, pre, D, n, io, ws, s);
         else xr::dispatch_sino_prefix<xr::GEO_PAR>(at, pre, D, n, io, ws, s);
     }
-    if (kind == xr::GEO_FLAT) xr::dispatch_gather<xr::GEO_FLAT>(rt, R, big, KC, gs, D, n, io, ws, s);
-    else if (kind == xr::GEO_ARC) xr::dispatch_gather<xr::GEO_ARC>(rt, R, big, KC, gs, D, n, io, ws, s);
-    else xr::dispatch_gather<xr::GEO_PAR>(rt, R, big, KC, gs, D, n, io, ws, s);
+    if (kind == xr::GEO_FLAT) xr::dispatch_gather<xr::GEO_FLAT>(rt, R, big, KC, fit, gs, D, n, io, ws, s);
+    else if (kind == xr::GEO_ARC) xr::dispatch_gather<xr::GEO_ARC>(rt, R, big, KC, fit, gs, D, n, io, ws, s);
+    else xr::dispatch_gather<xr::GEO_PAR>(rt, R, big, KC, fit, gs, D, n, io, ws, s);
     if (g_sum > 0) {
         const xr::BlockStarts sum =
             xr::block_starts(b->desc, [](const BatchDesc &d) { return xr::blocks_split_sum(d); });

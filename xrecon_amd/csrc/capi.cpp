@@ -100,7 +100,7 @@ void free_tables(Plan3d &p)
     if (p.d_lineC) (void)hipFree(p.d_lineC);
     if (p.d_lineV) (void)hipFree(p.d_lineV);
     if (p.d_col) (void)hipFree(p.d_col);
-    if (p.d_dcol) (void)hipFree(p.d_dcol);
+    if (p.d_cols) (void)hipFree(p.d_cols);
     if (p.d_vtile) (void)hipFree(p.d_vtile);
     if (p.d_cgrp) (void)hipFree(p.d_cgrp);
     if (p.d_citems) (void)hipFree(p.d_citems);
@@ -108,7 +108,7 @@ void free_tables(Plan3d &p)
     if (p.d_cqstage) (void)hipFree(p.d_cqstage);
     p.d_hdr = nullptr;
     p.d_lineC = p.d_lineV = p.d_col = nullptr;
-    p.d_dcol = nullptr;
+    p.d_cols = nullptr;
     p.d_vtile = nullptr;
     p.d_cgrp = nullptr;
     p.d_citems = nullptr;
@@ -148,7 +148,7 @@ int xr_plan3d_create(const xr_volume3d *vol, const xr_geometry3d *geo, const flo
     if (rc) return fail(rc, err);
     DeviceGuard g(device);
     if ((rc = upload(&p.d_hdr, t.hdr)) || (rc = upload(&p.d_lineC, t.lineC)) || (rc = upload(&p.d_lineV, t.lineV)) ||
-        (rc = upload(&p.d_col, t.col)) || (rc = upload(&p.d_dcol, t.dcol)) || (rc = upload(&p.d_vtile, t.vtile)) ||
+        (rc = upload(&p.d_col, t.col)) || (rc = upload(&p.d_cols, t.cols)) || (rc = upload(&p.d_vtile, t.vtile)) ||
         (rc = upload(&p.d_cgrp, t.cgrp)) || (rc = upload(&p.d_citems, t.citems)) ||
         (rc = upload(&p.d_cquad, t.cquad)) || (rc = upload(&p.d_cqstage, t.cqstage))) {
         free_tables(p);

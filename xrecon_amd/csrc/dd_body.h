@@ -8,6 +8,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <atomic>
 #include <cmath>
 #include <cstdint>
@@ -23,6 +24,9 @@ enum SinoMode : int { SINO_PLAIN = 0, SINO_AT = 1 };
 constexpr int kWave = 64;
 constexpr int kBlock = 256;
 constexpr int kWavesPerBlock = kBlock / kWave;
+
+// Entries after the last column in the tables read several columns at a time.
+constexpr int kColPad = 4;
 
 // Voxel-gather workgroup: a kVoxTile x kVoxTile block of voxel columns, each wave an
 // 8 x 8 tile of it.  The 64 lanes of a wave then project onto a compact detector patch
@@ -92,6 +96,18 @@ __host__ __device__ inline T g_load(const T *p)
 #endif
 }
 
+// N consecutive floats from a 4-byte aligned place, as one load.
+template <int N>
+__device__ inline void load_floats(const char *base, unsigned off, float *dst)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    typedef float vec __attribute__((ext_vector_type(N), aligned(4)));
+    const vec r = *(const __attribute__((address_space(1))) vec *)((const __attribute__((address_space(1))) char *)base + off);
+#pragma unroll
+    for (int i = 0; i < N; ++i) dst[i] = r[i];
+#endif
+}
+
 // The first three words {d, sigma, kappa} of a column-table entry (w = 0): what the voxel
 // gathers use of it, as one 12-byte load.
 __host__ __device__ inline float4 col_load3(const float4 *p)
@@ -128,6 +144,7 @@ struct VoxArgs {
     float hscale;  // dvv / dz
     int vsplit;    // view sets: set s sums views [s * vper, min(V, (s + 1) * vper))
     int vper;
+    int b0;        // first batch item of the launch
 };
 
 struct SinoArgs {
@@ -217,24 +234,50 @@ inline int default_rows(const Plan3d &p)
     return 1;
 }
 
-// Voxel-gather chunk: slices per thread in the low bits, XR_VOXEL_HALVES for chunks run
-// as two wave-culled halves (16 slices: halves of 8; 32 slices: halves of 16).  Halves
-// pay where many chunks straddle the detector's edge rows, and 32-slice chunks halve the
-// per-view work per slice (column search, weights, staging) on volumes tall enough to
-// keep the GPU busy: B per item of the 512^2 x 256 cone-arc workload 32.1 ms (16), 28.4
-// (16 in halves), 23.4 (32 in halves); on 256^2 x 64 plain 16-slice chunks win (2.71 /
-// 2.85 / 2.99 ms).  The autotuner tries every form.
+// Voxel-gather chunk: slices per thread in the low bits (XR_VOXEL_HALVES says nothing
+// further: every chunk passes over the slice groups off the detector).
 inline int chunk_slices(int k) { return k & 0xff; }
-inline bool chunk_halves(int k) { return (k & XR_VOXEL_HALVES) != 0; }
 
-inline int default_chunk(const Plan3d &p)
+// Plan3d::vox_fit bit of chunks of KC slices of NI items.
+inline int vox_fit_bit(int KC, int NI)
+{
+    const int k = KC >= 32 ? 2 : KC == 16 ? 1 : 0;
+    return 1 << (NI == 2 ? 3 + k : k);
+}
+
+// Workgroups of a voxel gather over nitem items (or pairs of them) in chunks of KC slices.
+inline int64_t vox_groups(const Plan3d &p, int KC, int64_t nitem)
+{
+    return (int64_t)ceil_div(p.vol.nx, kVoxTile) * ceil_div(p.vol.ny, kVoxTile) * ceil_div(p.vol.nz, KC) * p.vsplit * nitem;
+}
+
+// Whether chunks of KC slices (8 or 16) take two items per workgroup: where their blocks
+// fit the LDS and the pairs still fill the GPU (5 workgroups per CU are resident; 48^2 x 12,
+// 3 items, 700 views: 321 us in a pair and a single, 168 in singles of 8 slices).
+constexpr int64_t kVoxPairMin = 2048;
+inline bool vox_pairs(const Plan3d &p, int KC, int nbatch)
+{
+    return nbatch > 1 && (p.vox_fit & vox_fit_bit(KC, 2)) && vox_groups(p, KC, nbatch / 2) >= kVoxPairMin;
+}
+
+// The default chunk.  Several items: 16 slices of two instead of 32 of one (512^2 x 256
+// cone-arc A^T 15.1 ms per item against 19.1).  32 outputs per thread halve the per-view
+// work per output (line entry, column search, staging); with one item that pays on tall
+// volumes (512^2 x 256 A^T 19.1 ms against 18.9 with 16 slices, B 19.6 / 19.6, fewer
+// copies).  Up to 8 slices the places of a longer chunk that stay empty cost more than
+// they save (192^2, 360 views: 8 slices 142 / 139 us, 12 slices 206 / 168 with chunks of 8 /
+// 16), and so do chunks of 16 on grids too small to fill the GPU (80^2 x 20, 700 views, 800
+// workgroups: 142 / 159 us; 48^2 x 90, 864: 261 / 212).  Blocks that do not fit the LDS
+// cost more than shorter chunks do.
+constexpr int64_t kVoxTallMin = 832;
+inline int default_chunk(const Plan3d &p, int nbatch = 1)
 {
     const int nz = p.vol.nz;
-    if (nz >= 128) return 32 | XR_VOXEL_HALVES;
-    if (nz >= 64) return 16;
-    if (nz >= 8) return 8;
-    if (nz >= 4) return 4;
-    return 1;
+    if (nz > 8 && vox_pairs(p, 16, nbatch)) return 16;
+    int k = nz >= 128 ? 32 : nz > 8 ? 16 : nz > 1 ? 8 : 1;
+    for (; k > 8; k /= 2)
+        if ((p.vox_fit & vox_fit_bit(k, 1)) && vox_groups(p, k, nbatch) >= kVoxTallMin) break;
+    return k == 32 ? 32 | XR_VOXEL_HALVES : k;
 }
 
 inline bool valid_rows(int r) { return r == 1 || r == 2 || r == 4 || r == 8 || r == 16; }
@@ -269,6 +312,7 @@ inline VoxArgs make_vox_args(const Plan3d &p, int nbatch, int KC)
     a.hscale = p.dvv / p.dz;
     a.vsplit = p.vsplit;
     a.vper = (p.nview + p.vsplit - 1) / p.vsplit;
+    a.b0 = 0;
     return a;
 }
 
@@ -351,6 +395,39 @@ __host__ __device__ inline unsigned mad24(unsigned a, unsigned b, unsigned c)
 #endif
 }
 
+// The same with b the same on every lane of the wave.
+__host__ __device__ inline unsigned mad24_uniform(unsigned a, unsigned b, unsigned c)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    unsigned r;
+    asm("v_mad_u32_u24 %0, %1, %2, %3" : "=v"(r) : "v"(a), "s"(b), "v"(c));
+    return r;
+#else
+    return a * b + c;
+#endif
+}
+
+// acc = a * b + acc in place: the accumulators keep their registers across the branches of
+// a long loop body.
+__host__ __device__ inline void fmac(float &acc, float a, float b)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm("v_fmac_f32 %0, %1, %2" : "+v"(acc) : "v"(a), "v"(b));
+#else
+    acc = fmaf(a, b, acc);
+#endif
+}
+
+// A uniform value the compiler takes as new at this place, so that it does not keep
+// results derived from it (a scalar register pair per branch condition) across a loop.
+__host__ __device__ inline unsigned fresh(unsigned x)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("" : "+s"(x));
+#endif
+    return x;
+}
+
 // Two consecutive float2 table entries (pixels m and m+1 of a line) in one 16-byte load.
 // The entries are only 8-byte aligned, which gfx950 vector memory accesses allow.
 struct __attribute__((aligned(8))) Pair2 {
@@ -362,15 +439,24 @@ struct __attribute__((aligned(8))) Pair2 {
 // nothing staged.  Voxel gather: a view's row-prefix table (columns = detector columns,
 // rows = detector rows); skip = 1: no voxel of the workgroup's tile and slice chunk
 // reaches the detector on this view (bounds, not estimates: see VoxTile), so the
-// workgroup passes over the view.  Cell gather: a line of the z-prefix table (columns =
-// pixels along the line, rows = slices); skip unused.
+// workgroup passes over the view; off, in: bit g set when no voxel of slice group g
+// reaches the detector, or all of its rows lie inside it (bounds as well); full = 1: the
+// block holds every row the tile can look up.  Cell gather: a line of the z-prefix table
+// (columns = pixels along the line, rows = slices); skip, off, in and full unused.
 struct VoxBox {
     int c0, nc, r0, nr, pitch, skip;
+    unsigned off, in;
+    int full;
 };
 
+// Slices per group of the voxel gather (see voxel_column).
+constexpr int kVoxGroup = 4;
+__host__ __device__ constexpr int vox_group(int KC) { return KC < kVoxGroup ? KC : kVoxGroup; }
+
 #if !defined(__HIP_DEVICE_COMPILE__)
-// Host builds: staged cell-gather lookups found outside their LDS block (cell_line).
-inline std::atomic<long long> cell_box_misses{0};
+// Host builds: staged cell-gather lookups found outside their LDS block (cell_line); voxel
+// lookups off the detector or outside a block said to hold them (voxel_lookups).
+inline std::atomic<long long> cell_box_misses{0}, vox_box_misses{0};
 #endif
 
 // A float2 at byte offset off of an LDS block / of a table in global memory.  On the
@@ -427,6 +513,17 @@ __host__ __device__ inline float approx_rcp(float y)
 #endif
 }
 
+// 1 / y to within an ulp: v_rcp_f32 and one Newton step on the device.
+__host__ __device__ inline float near_rcp(float y)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    const float r = __builtin_amdgcn_rcpf(y);
+    return fmaf(fmaf(-y, r, 1.0f), r, r);
+#else
+    return 1.0f / y;
+#endif
+}
+
 // x / y where the quotient only seeds a search that is corrected against exact tables:
 // x times v_rcp_f32(y) on the device (about 2 ulp), a true division on the host.
 __host__ __device__ inline float seed_div(float x, float y)
@@ -447,10 +544,10 @@ __host__ __device__ inline float fdk_weight(float sx, float sy, float px, float 
         // sod^2 / (sod - (s.p)/sod)^2 written as 1 / (1 - (s.p)/sod^2)^2: one division per
         // call (1/sod^2 is loop-invariant and hoisted)
         const float t = fmaf(-(sx * px + sy * py), 1.0f / (sod * sod), 1.0f);
-        return 1.0f / (t * t);
+        return near_rcp(t * t);
     } else if (GEO == GEO_ARC) {
         const float ex = sx - px, ey = sy - py;
-        return 1.0f / (ex * ex + ey * ey);
+        return near_rcp(ex * ex + ey * ey);
     }
     return 1.0f;
 }
@@ -1009,6 +1106,34 @@ __host__ __device__ inline void cell_line_staged(CellLane<R> &st, const ViewHdr 
 
 // ---------------------------------------------------------------- voxel gather
 
+// True on every lane if the predicate holds on any active lane of the wave (device); the
+// predicate itself on the host, where each thread runs alone.
+__host__ __device__ inline bool wave_any(bool p)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_amdgcn_ballot_w64(p) != 0;
+#else
+    return p;
+#endif
+}
+
+// atan(t) where it only seeds a search that is corrected against exact tables: on the
+// device a least-squares odd polynomial for |t| <= 0.6 (within 3e-7; fans of up to 62
+// degrees), atanf beyond.
+__host__ __device__ inline float seed_atan(float t)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    if (wave_any(fabsf(t) > 0.6f)) return atanf(t);
+    const float q = t * t;
+    float r = fmaf(q, 0.0563796f, -0.1275247f);
+    r = fmaf(q, r, 0.1980930f);
+    r = fmaf(q, r, -0.3332516f);
+    return fmaf(t * q, r, t);
+#else
+    return atanf(t);
+#endif
+}
+
 // First column index to visit for axis point a: the closed-form inverse of the column map
 // (projective for flat and parallel, atan of a projective for arc).  A seed only: callers
 // correct it against the exact FP32 table.
@@ -1016,15 +1141,28 @@ template <int GEO>
 __host__ __device__ inline float column_seed(const ViewHdr &h, float a)
 {
     const float T = seed_div(fmaf(h.tp1, a, h.tp0), fmaf(h.tq1, a, h.tq0));
-    return h.tk0 + h.tk1 * (GEO == GEO_ARC ? atanf(T) : T);
+    return h.tk0 + h.tk1 * (GEO == GEO_ARC ? seed_atan(T) : T);
 }
 
 
-// Capacity of the staged block, in float2 entries (20 KiB of LDS per workgroup; 40 KiB
-// for chunks of 32 slices).  The blocks of 16 x 16 voxel columns x 16 slices of a 1 mm
-// volume seen by a 0.5 mm (at the isocentre) detector stay below 2400 entries.
-constexpr int kVoxLds = 2560;
-__host__ __device__ constexpr int vox_lds(int KC) { return KC >= 32 ? 2 * kVoxLds : kVoxLds; }
+// Capacity of the staged block, in float2 entries per item.  A workgroup waits for its
+// copies on every view, so resident workgroups decide the rate (256^2 x 64 cone-flat A^T
+// with 16 slices: 2.29 ms with 4 workgroups per CU, 1.51 with 6): 20 to 26 KiB for the 6
+// that 80 registers allow (8 and 16 slices), 30 KiB for the 5 of 96 registers (32 slices,
+// pairs of items).  The blocks of 16 x 16 voxel columns x 16 slices of a 1 mm volume seen by
+// a 0.5 mm (at the isocentre) detector of 64 rows stay below 2400 entries.
+__host__ __device__ constexpr int vox_lds(int KC, int NI = 1)
+{
+    return NI == 2 ? 1920 : KC >= 32 ? 3840 : KC == 16 ? 3328 : 2560;
+}
+// The general path copies whole rounds of pairs (voxel_stage): its buffers hold them.
+__host__ __device__ constexpr int vox_lds_rounds(int KC, int NI)
+{
+    return (vox_lds(KC, NI) + 2 * kBlock - 1) / (2 * kBlock) * (2 * kBlock);
+}
+// Widest block row: voxel_wg finds the place of pair p < 2^12 in a block of half pairs per
+// row as p ceil(2^20 / half) >> 20, exact while p half < 2^20.
+constexpr int kVoxMaxPitch = 512;
 
 // VoxTile for voxel columns [i0, i1] x [j0, j1] on view v, from the tile's corner pixels:
 // the axis map of a pixel edge is monotone in the pixel and in the line (a projective
@@ -1074,10 +1212,36 @@ inline VoxTile voxel_tile(const ViewHdr &h, const float4 *lineV, const float4 *c
 // one row outside [0, Nv] over the tile's whole depth-scale range (a voxel lane then fails
 // its own test rhi > 0 && rlo < Nv on every column: rounding moves its rows by far less
 // than a row).
+//
+// The slice groups' flags come from the rows of every slice boundary over the tile's
+// depth-scale range; a margin far above the rounding of a lane's row keeps them on the
+// safe side.
 template <int KC>
+__host__ __device__ inline void voxel_groups(const VoxTile &t, const VoxArgs &a, int k0, VoxBox &bx)
+{
+    constexpr int G = vox_group(KC);
+    const float fnv = (float)a.nv, mg = fmaf(1e-5f, fnv, 0.01f);
+    bx.off = bx.in = 0;
+    float lo = 0.0f, hi = 0.0f;
+#pragma unroll
+    for (int g = 0; g <= KC / G; ++g) {
+        const float z = fmaf((float)(k0 + g * G) - a.kmid, a.dz, a.zc), p = z * t.zk_lo, q = z * t.zk_hi;
+        const float l1 = fminf(p, q) - a.rv0, h1 = fmaxf(p, q) - a.rv0;
+        if (g > 0) {  // the group between boundaries (lo, hi) and (l1, h1)
+            const unsigned m = 1u << (g - 1);
+            if (!(h1 > -mg && lo < fnv + mg) || k0 + (g - 1) * G >= a.nz) bx.off |= m;
+            if (lo >= mg && h1 <= fnv - mg) bx.in |= m;
+        }
+        lo = l1;
+        hi = h1;
+    }
+    (void)hi;
+}
+
+template <int KC, int NI = 1>
 __host__ __device__ inline VoxBox voxel_box(const VoxTile &t, const VoxArgs &a, int k0)
 {
-    VoxBox bx{0, 0, 0, 0, 0, 0};
+    VoxBox bx{0, 0, 0, 0, 0, 0, 0, 0, 0};
     if (t.nc < 0) bx.skip = 1;
     if (t.nc <= 0) return bx;
     const float zlo = fmaf((float)k0, a.dz, a.zb), zhi = fmaf((float)(k0 + KC), a.dz, a.zb);
@@ -1093,9 +1257,11 @@ __host__ __device__ inline VoxBox voxel_box(const VoxTile &t, const VoxArgs &a, 
     const int r1 = imin((int)floorf(hi) + 1, a.nv);
     const int pitch = (t.nc + 1) & ~1;
     int nr = r1 - r0 + 1;
-    constexpr int cap = vox_lds(KC);
-    if (nr <= 0 || pitch > cap) return bx;
-    if (pitch * nr > cap) nr = cap / pitch;
+    constexpr int cap = vox_lds(KC, NI);
+    voxel_groups<KC>(t, a, k0, bx);
+    if (nr <= 0 || pitch > cap || pitch > kVoxMaxPitch) return bx;
+    bx.full = pitch * nr <= cap;
+    if (!bx.full) nr = cap / pitch;
     bx.c0 = t.c0;
     bx.nc = t.nc;
     bx.r0 = r0;
@@ -1151,22 +1317,11 @@ __host__ __device__ inline void voxel_stage(const float2 *__restrict__ Qv, const
     }
 }
 
-// True on every lane if the predicate holds on any active lane of the wave (device); the
-// predicate itself on the host, where each thread runs alone.
-__host__ __device__ inline bool wave_any(bool p)
-{
-#if defined(__HIP_DEVICE_COMPILE__)
-    return __builtin_amdgcn_ballot_w64(p) != 0;
-#else
-    return p;
-#endif
-}
-
-
 // Where one column's row-prefix entries are read from: the staged LDS block (when the
 // column lies in it) or the view's table in HBM.  Lb is the LDS block itself (never
 // replaced by a null pointer: a pointer that may be either would compile to generic
-// "flat" loads for the LDS reads); in_lds says whether this column is staged.
+// "flat" loads for the LDS reads); in_lds says whether this column is staged.  Item it of
+// a thread's items reads the block it * lds_item and the table it * q_item bytes further.
 struct VoxCol {
     const char *Qb;   // view's table
     unsigned nu8;     // byte stride of a table row
@@ -1176,69 +1331,137 @@ struct VoxCol {
     unsigned lcb;     // (c - c0) * 8 - r0 * pitch * 8: LDS byte offset of row 0 (mod 2^32)
     unsigned nc8;     // LDS row pitch in bytes
     int r0, r1;       // staged rows [r0, r1)
+    unsigned lds_item;
+    int64_t q_item;
 };
 
-// Slice boundaries q = Q0..Q1 of one column: rows rho_q = clamp(rlo + q step, 0, Nv), one
-// row-prefix lookup each, I(rho) = B_r + rho p_r; accumulates slices Q0..Q1-1 with weight
-// w and returns I at boundary Q1.  With have_first the caller already holds I at Q0
-// (Ifirst) and that lookup is not repeated.  All lookups are independent: the rows are
-// computed, the loads issued back to back, then consumed.
-template <int Q0, int Q1>
-__host__ __device__ inline float voxel_slices(const VoxCol &cs, float rlo, float step, float fnv, float w,
-                                              bool have_first, float Ifirst, float *acc)
+// The row-prefix integrals I(rho) = B_r + rho p_r of one column at the N rows rh (clamped
+// to the detector where CLAMP; the caller knows that they lie on it otherwise), for every
+// item.  FULL: every lookup lies in the staged block.  All lookups are independent: the
+// loads are issued back to back, then consumed.
+template <int N, int NI, bool CLAMP, bool FULL>
+__host__ __device__ inline void voxel_lookups(const VoxCol &cs, float *rh, float fnv, float (*I)[N])
 {
-    constexpr int N = Q1 - Q0;
-    int ri[N + 1];
-    float rh[N + 1];
-#pragma unroll
-    for (int q = 0; q <= N; ++q) {
-        rh[q] = clampf(fmaf((float)(Q0 + q), step, rlo), 0.0f, fnv);
-        ri[q] = (int)rh[q];
-    }
-    float2 e[N + 1];
-    // rows increase with q, so the first and last lookups bound the span's rows
-    const bool staged = cs.in_lds && ri[0] >= cs.r0 && ri[N] < cs.r1;
-    if (staged) {
-        // byte offset (ri - r0) * pitch * 8 + (c - c0) * 8 as one 24-bit multiply-add
-        // (unsigned wrap-around of the constant part is exact)
-        if (!have_first) e[0] = lds_float2(cs.Lb, mad24((unsigned)ri[0], cs.nc8, cs.lcb));
-#pragma unroll
-        for (int q = 1; q <= N; ++q) e[q] = lds_float2(cs.Lb, mad24((unsigned)ri[q], cs.nc8, cs.lcb));
-    } else {
-        if (!have_first) e[0] = global_float2(cs.Qb, mul24((unsigned)ri[0], cs.nu8) + cs.c8);
-#pragma unroll
-        for (int q = 1; q <= N; ++q) e[q] = global_float2(cs.Qb, mul24((unsigned)ri[q], cs.nu8) + cs.c8);
-    }
-    // I(rho) = B_r + rho q_r (see prefix_column)
-    float Ip = have_first ? Ifirst : fmaf(rh[0], e[0].y, e[0].x);
+    int ri[N];
 #pragma unroll
     for (int q = 0; q < N; ++q) {
-        const float In = fmaf(rh[q + 1], e[q + 1].y, e[q + 1].x);
-        acc[Q0 + q] = fmaf(w, In - Ip, acc[Q0 + q]);
-        Ip = In;
+        if (CLAMP) rh[q] = clampf(rh[q], 0.0f, fnv);
+        ri[q] = (int)rh[q];
     }
-    return Ip;
+#if !defined(__HIP_DEVICE_COMPILE__)
+    for (int q = 0; q < N; ++q)
+        if (!(rh[q] >= 0.0f && rh[q] <= fnv) || (FULL && !(cs.in_lds && ri[q] >= cs.r0 && ri[q] < cs.r1)))
+            vox_box_misses.fetch_add(1);
+#endif
+    float2 e[NI][N];
+    // rows increase with q, so the first and last lookups bound the span's rows
+    if (FULL || (cs.in_lds && ri[0] >= cs.r0 && ri[N - 1] < cs.r1)) {
+        // byte offset (ri - r0) * pitch * 8 + (c - c0) * 8 as one 24-bit multiply-add
+        // (unsigned wrap-around of the constant part is exact)
+#pragma unroll
+        for (int q = 0; q < N; ++q) {
+            const unsigned off = mad24_uniform((unsigned)ri[q], cs.nc8, cs.lcb);
+#pragma unroll
+            for (int it = 0; it < NI; ++it) e[it][q] = lds_float2(cs.Lb + it * cs.lds_item, off);
+        }
+    } else {
+#pragma unroll
+        for (int q = 0; q < N; ++q) {
+            const unsigned off = mul24((unsigned)ri[q], cs.nu8) + cs.c8;
+#pragma unroll
+            for (int it = 0; it < NI; ++it) e[it][q] = global_float2(cs.Qb + it * cs.q_item, off);
+        }
+    }
+#pragma unroll
+    for (int it = 0; it < NI; ++it)
+#pragma unroll
+        for (int q = 0; q < N; ++q) I[it][q] = fmaf(rh[q], e[it][q].y, e[it][q].x);
 }
 
-// One view's contribution to the KC slice accumulators of voxel column (i, j).  With a
-// staged block (lds != nullptr), lookups inside it read LDS, the rest the table in HBM.
-//
-// With HALVES, chunks of 16 slices run as two halves of 8, each skipped when no lane of
-// the wave has a row of that half on the detector: every boundary of a skipped half then
-// clamps to the same row (0 below, Nv above) for every lane, so its differences are
-// exactly zero and skipping it changes no result.
-template <int OPK, int GEO, int KC, bool HALVES = false>
-__host__ __device__ inline void voxel_view(const ViewHdr &h, const float4 *__restrict__ lineV,
-                                           const float4 *__restrict__ ct, const float2 *__restrict__ Qv,
-                                           const VoxArgs &a, int v, int i, int j, int k0, float px, float py,
-                                           float *acc, const VoxBox &bx, const float2 *__restrict__ lds)
+// Slices g G .. g G + G - 1 of one column: boundary rows from the group's first, and the
+// last from the next group's first, so that a boundary's row does not depend on the chunk.
+template <int KC, int NI, int G, bool CLAMP, bool FULL>
+__host__ __device__ inline void voxel_group(const VoxCol &cs, int g, float first, float next, float step, float fnv,
+                                            float w, float *Ip, float *acc)
 {
-    static_assert(KC <= 16 || HALVES, "chunks beyond 16 slices run in halves");
+    float rh[G], I[NI][G];
+#pragma unroll
+    for (int q = 1; q < G; ++q) rh[q - 1] = fmaf((float)q, step, first);
+    rh[G - 1] = next;
+    voxel_lookups<G, NI, CLAMP, FULL>(cs, rh, fnv, I);
+#pragma unroll
+    for (int it = 0; it < NI; ++it)
+#pragma unroll
+        for (int q = 0; q < G; ++q) {
+            fmac(acc[it * KC + g * G + q], w, I[it][q] - Ip[it]);
+            Ip[it] = I[it][q];
+        }
+}
+
+// One column's contribution, weight w, to the KC slices of NI items (acc[it * KC + q]):
+// slice boundary k lies at row kf step + base, kf the boundary measured from the volume's
+// middle (kf[g]: group g's first).
+// The slices go in groups of kVoxGroup, whose flags (VoxBox::off, in) are the same for the
+// whole workgroup: a group off the detector is passed over (every boundary would clamp to
+// the same row, its differences are exactly zero), one inside it needs no clamp.  The
+// 256^2 x 64 cone-flat volume is twice as tall as the field of view: 58 % of the lookups
+// of 16-slice chunks fell on the detector.
+template <int KC, int NI, bool FULL>
+__host__ __device__ inline void voxel_column(const VoxCol &cs, const VoxBox &bx, const float *kf, float step,
+                                             float base, float fnv, float w, float *acc)
+{
+    constexpr int G = vox_group(KC);
+    float Ip[NI];
+    const unsigned off = fresh(bx.off), in = fresh(bx.in);
+#pragma unroll
+    for (int g = 0; g < KC / G; ++g) {
+        if (off & (1u << g)) continue;
+        const float first = fmaf(kf[g], step, base), next = fmaf(kf[g + 1], step, base);
+        if (g == 0 || (off & (1u << (g - 1)))) {
+            float rh[1] = {first}, I[NI][1];
+            voxel_lookups<1, NI, true, FULL>(cs, rh, fnv, I);
+#pragma unroll
+            for (int it = 0; it < NI; ++it) Ip[it] = I[it][0];
+        }
+        if (in & (1u << g)) voxel_group<KC, NI, G, false, FULL>(cs, g, first, next, step, fnv, w, Ip, acc);
+        else voxel_group<KC, NI, G, true, FULL>(cs, g, first, next, step, fnv, w, Ip, acc);
+    }
+}
+
+// First boundary of every slice group of a chunk (and the chunk's last) measured from the
+// volume's middle, in slices (the same for the whole workgroup: kept in scalar registers).
+template <int KC>
+__host__ __device__ inline void voxel_kf(const VoxArgs &a, int k0, float *kf)
+{
+    constexpr int G = vox_group(KC);
+#pragma unroll
+    for (int g = 0; g <= KC / G; ++g) {
+        const float x = (float)(k0 + g * G) - a.kmid;
+#if defined(__HIP_DEVICE_COMPILE__)
+        kf[g] = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, x)));
+#else
+        kf[g] = x;
+#endif
+    }
+}
+
+// One view's contribution to the KC slice accumulators of voxel column (i, j) of NI items
+// (item it: acc + it * KC, the table Qv + it * q_item and the block lds + it * vox_lds_rounds(KC, NI)),
+// from the line entry lv and the group boundaries kf.  With a staged block (lds !=
+// nullptr), lookups inside it read LDS, the rest the table in HBM.
+template <int OPK, int GEO, int KC, int NI>
+__host__ __device__ inline void voxel_view_items(const ViewHdr &h, const float4 &lv, const float4 *__restrict__ ct,
+                                                 const float2 *__restrict__ Qv, int64_t q_item, const VoxArgs &a,
+                                                 int m, const float *kf, float px, float py, float *acc,
+                                                 const VoxBox &box, const float2 *__restrict__ lds)
+{
     const float fnv = (float)a.nv;
     const int nu = a.nu;
-    int L, m;
-    if (h.xdrv) { L = j; m = i; } else { L = i; m = a.ny - 1 - j; }
-    const float4 lv = g_load(lineV + (int64_t)v * a.maxline + L);  // {P0, Delta, zeta, 1/(Delta zeta)}
+    VoxBox bx = box;  // (the same on every lane)
+    bx.off = (unsigned)wave_uniform((int)box.off);
+    bx.in = (unsigned)wave_uniform((int)box.in);
+    bx.full = wave_uniform(box.full);
+    bx.pitch = wave_uniform(box.pitch);
     const float a0 = fmaf((float)m, lv.y, lv.x);
     const float a1 = a0 + lv.y;
     if (!(a1 > h.dlo && a0 < h.dhi)) return;
@@ -1269,6 +1492,7 @@ __host__ __device__ inline void voxel_view(const ViewHdr &h, const float4 *__res
     const char *Qb = reinterpret_cast<const char *>(Qv);
     const unsigned nu8 = (unsigned)nu * 8u;
     const unsigned nc8 = (unsigned)bx.pitch * 8u;
+    const unsigned row0 = (unsigned)bx.c0 * 8u + (unsigned)bx.r0 * nc8;
     const char *ctb = reinterpret_cast<const char *>(ct);
     while (c < nu && cc.x < a1) {
         // prefetch the next column's table entry one iteration ahead (32-bit byte offset
@@ -1280,32 +1504,99 @@ __host__ __device__ inline void voxel_view(const ViewHdr &h, const float4 *__res
             const float kap = cc.z;
             const float step = zsz * kap;
             const float base = fmaf(zcz, kap, -a.rv0);
-            const float rlo = fmaf((float)k0 - a.kmid, step, base);
-            const float rhi = fmaf((float)(k0 + KC) - a.kmid, step, base);
-            if (rhi > 0.0f && rlo < fnv) {
-                // B: ou * U w sigma dvv / (Delta zeta dz); A^T: ou (normalisation folded
-                // into the prefix table).
-                const float w = (OPK == VOX_AT) ? ou : ou * hB * cc.y;
-                const bool in_lds = lds != nullptr && (unsigned)(c - bx.c0) < (unsigned)bx.nc;
-                const VoxCol cs{Qb, nu8, (unsigned)c * 8u, reinterpret_cast<const char *>(lds), in_lds,
-                                (unsigned)(c - bx.c0) * 8u - (unsigned)bx.r0 * nc8, nc8, bx.r0, bx.r0 + bx.nr};
-                if (!HALVES || KC < 16) {
-                    voxel_slices<0, KC>(cs, rlo, step, fnv, w, false, 0.0f, acc);
-                } else {
-                    constexpr int H = KC / 2;
-                    const float rmid = fmaf((float)H, step, rlo);
-                    // this lane's lower half reaches row 0 iff rmid > 0 (its chunk starts
-                    // below Nv), the upper half iff rmid < Nv (its chunk ends above 0)
-                    const bool lo = wave_any(rmid > 0.0f), hi = wave_any(rmid < fnv);
-                    float Imid = 0.0f;
-                    if (lo) Imid = voxel_slices<0, H>(cs, rlo, step, fnv, w, false, 0.0f, acc);
-                    if (hi) voxel_slices<H, KC>(cs, rlo, step, fnv, w, lo, Imid, acc);
-                }
-            }
+            // B: ou * U w sigma dvv / (Delta zeta dz); A^T: ou (normalisation folded
+            // into the prefix table).
+            const float w = (OPK == VOX_AT) ? ou : ou * hB * cc.y;
+            const bool in_lds = lds != nullptr && (unsigned)(c - bx.c0) < (unsigned)bx.nc;
+            const VoxCol cs{Qb, nu8, (unsigned)c * 8u, reinterpret_cast<const char *>(lds), in_lds,
+                            (unsigned)c * 8u - row0, nc8, bx.r0, bx.r0 + bx.nr,
+                            (unsigned)(vox_lds_rounds(KC, NI) * sizeof(float2)), q_item * (int64_t)sizeof(float2)};
+            if (bx.full) voxel_column<KC, NI, true>(cs, bx, kf, step, base, fnv, w, acc);
+            else voxel_column<KC, NI, false>(cs, bx, kf, step, base, fnv, w, acc);
         }
         ++c;
         cc = cn;
         cn = cnn;
+    }
+}
+
+// The same for one item, from the tables.
+template <int OPK, int GEO, int KC, bool HALVES = false>
+__host__ __device__ inline void voxel_view(const ViewHdr &h, const float4 *__restrict__ lineV,
+                                           const float4 *__restrict__ ct, const float2 *__restrict__ Qv,
+                                           const VoxArgs &a, int v, int i, int j, int k0, float px, float py,
+                                           float *acc, const VoxBox &bx, const float2 *__restrict__ lds)
+{
+    const int L = h.xdrv ? j : i, m = h.xdrv ? i : a.ny - 1 - j;
+    float kf[KC / vox_group(KC) + 1];
+    voxel_kf<KC>(a, k0, kf);
+    voxel_view_items<OPK, GEO, KC, 1>(h, g_load(lineV + (int64_t)v * a.maxline + L), ct, Qv, 0, a, m, kf, px, py, acc,
+                                      bx, lds);
+}
+
+// What a voxel column needs of one view before its gather: its footprint [a0, a1] on the
+// axis, both ends on the detector (equal where it misses it), and the entries of the
+// first three columns from the one the closed-form inverse gives (corrected where it came
+// out past a0; columns before the footprint have no width).  cols: the view's boundaries d
+// (Nu + kColPad floats), then the row scales kappa, then the depth scales sigma.
+template <int OPK, int GEO>
+struct VoxelColumns {
+    float a0, a1, d[4], kap[3], sig[3];
+    int c;
+    __device__ void load(const float *cols, int nu)
+    {
+        const char *t = reinterpret_cast<const char *>(cols);
+        const int sp = nu + kColPad;
+        load_floats<4>(t, (unsigned)c * 4u, d);
+        load_floats<3>(t + (int64_t)sp * 4, (unsigned)c * 4u, kap);
+        if (OPK != VOX_AT) load_floats<3>(t + (int64_t)sp * 8, (unsigned)c * 4u, sig);
+    }
+    __device__ void start(const ViewHdr &h, const float4 &lv, int m, const float *cols, int nu, bool active)
+    {
+        const float e = fmaf((float)m, lv.y, lv.x);
+        a0 = clampf(e, h.dlo, h.dhi);
+        a1 = active ? clampf(e + lv.y, h.dlo, h.dhi) : a0;
+        c = (int)clampf(column_seed<GEO>(h, a0), 0.0f, (float)(nu - 1));
+        load(cols, nu);
+    }
+    __device__ void correct(const float *cols, int nu)
+    {
+        while (wave_any(d[0] > a0)) {  // (d_0 <= a0, so c stays above 0 here)
+            if (d[0] > a0) --c;
+            load(cols, nu);
+        }
+    }
+};
+
+// One view of voxel_wg: NI items' KC slices, every lookup in the staged blocks at lds.
+template <int OPK, int GEO, int KC, int NI>
+__device__ inline void voxel_view_staged(VoxelColumns<OPK, GEO> &vc, const ViewHdr &h, const float4 &lv,
+                                         const float *cols, const VoxArgs &a, const float *kf, float px, float py,
+                                         float *acc, const VoxBox &bx, const char *lds)
+{
+    const float fnv = (float)a.nv;
+    float hB = 1.0f;
+    if (OPK != VOX_AT) {
+        const float U = (OPK == VOX_BW) ? fdk_weight<GEO>(h.sx, h.sy, px, py, a.sod) : 1.0f;
+        hB = U * h.colw * a.hscale * lv.w;  // as in voxel_view_items
+    }
+    const float zcz = lv.z * a.zc, zsz = lv.z * a.dz;
+    const unsigned nc8 = (unsigned)bx.pitch * 8u, row0 = (unsigned)bx.c0 * 8u + (unsigned)bx.r0 * nc8;
+    for (;;) {
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            const float b = clampf(vc.d[q + 1], vc.a0, vc.a1), ou = b - vc.a0;
+            vc.a0 = b;
+            if (ou > 0.0f) {
+                const float w = (OPK == VOX_AT) ? ou : ou * hB * vc.sig[q];
+                const VoxCol cs{nullptr, 0, 0, lds, true, (unsigned)(vc.c + q) * 8u - row0, nc8, 0, 0,
+                                (unsigned)(vox_lds(KC, NI) * sizeof(float2)), 0};
+                voxel_column<KC, NI, true>(cs, bx, kf, zsz * vc.kap[q], fmaf(zcz, vc.kap[q], -a.rv0), fnv, w, acc);
+            }
+        }
+        if (!wave_any(vc.a0 < vc.a1)) break;
+        vc.c = imin(vc.c + 3, a.nu - 1);  // (a pixel that is done has no width left)
+        vc.load(cols, a.nu);
     }
 }
 
@@ -1340,53 +1631,11 @@ __host__ __device__ inline void voxel_body(const ViewHdr *__restrict__ hdr, cons
     const float px = voxel_px(a, i), py = voxel_py(a, j);
     float acc[KC];
     for (int q = 0; q < KC; ++q) acc[q] = 0.0f;
-    const VoxBox none{0, 0, 0, 0, 0, 0};
+    const VoxBox none{0, 0, 0, 0, 0, 0, 0, 0, 0};
     for (int v = v0; v < v1; ++v)
         voxel_view<OPK, GEO, KC, HALVES>(hdr[v], lineV, colt + (int64_t)v * (a.nu + 1), view_table(Q, a, b, v), a, v,
                                          i, j, k0, px, py, acc, none, nullptr);
     voxel_store<KC>(out, a, i, j, k0, b, acc);
-}
-
-// A workgroup of the voxel gather (device only): the 16 x 16 tile tile_id of voxel
-// columns, slices k0..k0+KC-1, batch b, views [v0, v1); this thread owns (i, j) when
-// `active`.  Per view the
-// workgroup stages the block of the row-prefix table its footprint reads into LDS, then
-// every thread gathers from it.  Inactive threads take part in staging and barriers.
-// (A second, alternating buffer that overlaps the next view's staging with this view's
-// gather measured slower: the gather's own table loads must wait for the earlier-issued
-// staging loads anyway, and the doubled code and registers cost more than they save.)
-// Chunks of fewer than kVoxStageMin slices read the table directly: a staged block then
-// serves too few lookups to repay its copy and the two barriers per view.
-constexpr int kVoxStageMin = 8;
-
-template <int OPK, int GEO, int KC, bool HALVES = false>
-__device__ inline void voxel_wg(const ViewHdr *__restrict__ hdr, const float4 *__restrict__ lineV,
-                                const float4 *__restrict__ colt, const VoxTile *__restrict__ vtile,
-                                const float2 *__restrict__ Q, float *__restrict__ out, const VoxArgs &a, int i, int j,
-                                bool active, int tile_id, int k0, int b, int v0, int v1,
-                                float2 *__restrict__ tile)
-{
-    if (KC < kVoxStageMin) {
-        if (active) voxel_body<OPK, GEO, KC, HALVES>(hdr, lineV, colt, Q, out, a, i, j, k0, b, v0, v1);
-        return;
-    }
-    const float px = voxel_px(a, i), py = voxel_py(a, j);
-    float acc[KC];
-    for (int q = 0; q < KC; ++q) acc[q] = 0.0f;
-    const int ntile = ceil_div(a.nx, kVoxTile) * ceil_div(a.ny, kVoxTile);
-    for (int v = v0; v < v1; ++v) {
-        const ViewHdr h = ro_load(hdr + v);
-        const float4 *ct = colt + (int64_t)v * (a.nu + 1);
-        const float2 *Qv = view_table(Q, a, b, v);
-        const VoxBox bx = voxel_box<KC>(ro_load(vtile + (int64_t)v * ntile + tile_id), a, k0);
-        if (bx.skip) continue;  // the same for every thread of the workgroup: no barrier is missed
-        voxel_stage(Qv, bx, tile, a.nu, threadIdx.x, kBlock);
-        __builtin_amdgcn_s_waitcnt(0);  // this wave's direct-to-LDS loads have landed
-        __syncthreads();
-        if (active) voxel_view<OPK, GEO, KC, HALVES>(h, lineV, ct, Qv, a, v, i, j, k0, px, py, acc, bx, tile);
-        __syncthreads();
-    }
-    if (active) voxel_store<KC>(out, a, i, j, k0, b, acc);
 }
 
 // Waits until at most n (0..4) of this wave's vector memory loads are outstanding (they
@@ -1414,6 +1663,179 @@ __device__ inline void wg_barrier()
     __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0) only
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
+}
+
+// Entries that the block of tile t can need for any chunk of KC slices (voxel_box): rows
+// over the chunk at the largest depth scale, plus the spread of the depth scale at the
+// outermost slice whose rows reach the detector, plus margins; 0 where nothing is staged.
+inline int64_t voxel_block_bound(const VoxTile &t, const VoxArgs &a, int KC)
+{
+    if (t.nc <= 0) return 0;
+    const double zmax = std::max(std::fabs((double)a.zb), std::fabs((double)a.zb + (double)a.nz * a.dz)) + KC * (double)a.dz;
+    const double reach = (std::max(std::fabs((double)a.rv0), std::fabs((double)a.rv0 + a.nv)) + 2.0) / std::max((double)t.zk_lo, 1e-30) +
+                         KC * (double)a.dz;
+    const double rows = KC * (double)a.dz * t.zk_hi + std::min(zmax, reach) * ((double)t.zk_hi - t.zk_lo) + 6.0;
+    const int64_t pitch = (t.nc + 1) & ~1;
+    if (pitch > kVoxMaxPitch) return INT64_MAX;
+    return pitch * (int64_t)std::min(rows, (double)a.nv + 1.0);
+}
+
+// Whether every block of tile t fits the LDS with chunks of KC slices of NI items.
+template <int KC, int NI>
+inline bool voxel_tile_fits(const VoxTile &t, const VoxArgs &a)
+{
+    if (voxel_block_bound(t, a, KC) <= vox_lds(KC, NI)) return true;
+    for (int k0 = 0; k0 < a.nz; k0 += KC) {
+        const VoxBox bx = voxel_box<KC, NI>(t, a, k0);
+        if (t.nc > 0 && !bx.skip && !bx.full) return false;
+    }
+    return true;
+}
+
+// A workgroup of the voxel gather (device only): the 16 x 16 tile tile_id of voxel
+// columns, slices k0..k0+KC-1, batch b, views [v0, v1); this thread owns (i, j) when
+// `active`.  Per view the
+// workgroup stages the block of the row-prefix table its footprint reads into LDS, then
+// every thread gathers from it.  Inactive threads take part in staging and barriers.
+// (A second, alternating buffer that overlaps the next view's staging with this view's
+// gather measured slower: the gather's own table loads must wait for the earlier-issued
+// staging loads anyway, and the doubled code and registers cost more than they save.)
+// Chunks of fewer than kVoxStageMin slices read the table directly: a staged block then
+// serves too few lookups to repay its copy and the two barriers per view.
+constexpr int kVoxStageMin = 8;
+
+//
+// Lane l of each wave works out the block of view base + l for 64 views at a time (read
+// back per view with readlane); views that the tile's chunk misses are never visited.
+//
+// FIT: every block of the plan fits the LDS (Plan3d::vox_fit); otherwise lookups outside
+// their block read the table, view by view with nothing worked out ahead.
+template <int OPK, int GEO, int KC, int NI, bool FIT>
+__device__ inline void voxel_wg(const ViewHdr *__restrict__ hdr, const float4 *__restrict__ lineV,
+                                const float4 *__restrict__ colt, const float *__restrict__ cols,
+                                const VoxTile *__restrict__ vtile, const float2 *__restrict__ Q,
+                                float *__restrict__ out, const VoxArgs &a, int i, int j, bool active, int tile_id,
+                                int k0, int b, int v0, int v1, float2 *__restrict__ tile)
+{
+    if constexpr (KC < kVoxStageMin) {
+        if (active) voxel_body<OPK, GEO, KC>(hdr, lineV, colt, Q, out, a, i, j, k0, b, v0, v1);
+        return;
+    }
+    const float px = voxel_px(a, i), py = voxel_py(a, j);
+    float acc[NI * KC], kf[KC / vox_group(KC) + 1];
+#pragma unroll
+    for (int q = 0; q < NI * KC; ++q) acc[q] = 0.0f;
+    voxel_kf<KC>(a, k0, kf);
+    const int ntile = ceil_div(a.nx, kVoxTile) * ceil_div(a.ny, kVoxTile);
+    const int64_t q_item = (int64_t)a.nview * (a.nv + 1) * a.nu;
+    const int tid = threadIdx.x, lane = tid & (kWave - 1);
+    const unsigned nu8 = (unsigned)a.nu * 8u;
+    const int64_t sp = 3 * (a.nu + kColPad);
+    const int ic = imin(i, a.nx - 1), jc = imin(j, a.ny - 1);
+    if constexpr (!FIT) {
+        for (int v = v0; v < v1; ++v) {
+            const ViewHdr h = ro_load(hdr + v);
+            const float2 *Qv = view_table(Q, a, b, v);
+            const VoxBox bx = voxel_box<KC, NI>(ro_load(vtile + (int64_t)v * ntile + tile_id), a, k0);
+            if (bx.skip) continue;  // the same for every thread of the workgroup: no barrier is missed
+            for (int it = 0; it < NI; ++it)
+                voxel_stage(Qv + it * q_item, bx, tile + it * vox_lds_rounds(KC, NI), a.nu, tid, kBlock);
+            const int xd = wave_uniform(h.xdrv);
+            const float4 lv = g_load(lineV + (int64_t)v * a.maxline + (xd ? jc : ic));
+            __builtin_amdgcn_s_waitcnt(0);  // this wave's direct-to-LDS loads have landed
+            __syncthreads();
+            if (active)
+                voxel_view_items<OPK, GEO, KC, NI>(h, lv, colt + (int64_t)v * (a.nu + 1), Qv, q_item, a,
+                                                   xd ? i : a.ny - 1 - j, kf, px, py, acc, bx, tile);
+            __syncthreads();
+        }
+        if (active) {
+#pragma unroll
+            for (int it = 0; it < NI; ++it) voxel_store<KC>(out, a, i, j, k0, b + it, acc + it * KC);
+        }
+        return;
+    }
+    for (int base = v0; base < v1; base += kWave) {
+        // the block of view base + lane, packed: rows and pitch < 2^13, groups < 2^8
+        int mc0, mr0, msize, mflags;
+        unsigned mplaces;
+        unsigned long long todo;
+        {
+            const VoxBox bx = voxel_box<KC, NI>(g_load(vtile + (int64_t)imin(base + lane, v1 - 1) * ntile + tile_id), a, k0);
+            const int half = imax(bx.pitch >> 1, 1);
+            mc0 = bx.c0;
+            mr0 = bx.r0;
+            msize = bx.nr << 16 | bx.pitch;
+            mflags = (int)(bx.off << 16 | bx.in);
+            mplaces = ((1u << 20) + half - 1) / half;
+            todo = __builtin_amdgcn_ballot_w64(!bx.skip && base + lane < v1);
+        }
+        if (!todo) continue;
+        // views, blocks and copies are the same for the whole workgroup
+        auto box_of = [&](int l) {
+            const int size = __builtin_amdgcn_readlane(msize, l), flags = __builtin_amdgcn_readlane(mflags, l);
+            VoxBox bx;
+            bx.c0 = __builtin_amdgcn_readlane(mc0, l);
+            bx.r0 = __builtin_amdgcn_readlane(mr0, l);
+            bx.nr = size >> 16;
+            bx.pitch = size & 0xFFFF;
+            bx.nc = bx.pitch;
+            bx.off = (unsigned)flags >> 16;
+            bx.in = (unsigned)flags & 0xFFFF;
+            bx.full = 1;
+            bx.skip = 0;
+            return bx;
+        };
+        auto stage = [&](int l, const VoxBox &bx) {  // as voxel_stage, pair p at row p / half of the block
+            const float2 *Qv = view_table(Q, a, b, base + l);
+            const unsigned pl = __builtin_amdgcn_readlane(mplaces, l);
+            const int half = bx.pitch >> 1, pairs = bx.nr * half;
+            const unsigned first = (unsigned)bx.r0 * nu8 + (unsigned)bx.c0 * 8u;
+            for (int s = 0; s * kBlock < pairs; ++s) {
+                const unsigned p = (unsigned)(tid + s * kBlock), r = mul24(p, pl) >> 20;
+                const unsigned off = mad24_uniform(r, nu8, (p - mul24(r, (unsigned)half)) * 16u + first);
+                float2 *dst = tile + 2 * (s * kBlock + (tid & ~(kWave - 1)));
+                if (p >= (unsigned)pairs) continue;  // (the block need not fill whole rounds)
+#pragma unroll
+                for (int it = 0; it < NI; ++it)
+                    __builtin_amdgcn_global_load_lds(reinterpret_cast<const char *>(Qv + it * q_item) + off,
+                                                     (__attribute__((address_space(3))) void *)(dst + it * vox_lds(KC, NI)),
+                                                     16, 0, 0);
+            }
+        };
+        auto line_of = [&](int v, const ViewHdr &h) {
+            return g_load(lineV + (int64_t)v * a.maxline + (wave_uniform(h.xdrv) ? jc : ic));
+        };
+        // A view's column entries load beside its copies; the next view's header and line
+        // entry load during its gather.
+        int l = __builtin_ctzll(todo);
+        ViewHdr h = ro_load(hdr + base + l);
+        float4 lv = line_of(base + l, h);
+        for (;;) {
+            todo &= todo - 1;
+            const VoxBox bx = box_of(l);
+            const float *cv = cols + (base + l) * sp;
+            VoxelColumns<OPK, GEO> vc;
+            vc.start(h, lv, wave_uniform(h.xdrv) ? ic : a.ny - 1 - jc, cv, a.nu, active);
+            stage(l, bx);
+            __builtin_amdgcn_s_waitcnt(0);  // this wave's direct-to-LDS loads have landed
+            wg_barrier();
+            const int ln = todo ? __builtin_ctzll(todo) : l;
+            const ViewHdr hn = ro_load(hdr + base + ln);
+            const float4 lvn = line_of(base + ln, hn);
+            vc.correct(cv, a.nu);
+            voxel_view_staged<OPK, GEO, KC, NI>(vc, h, lv, cv, a, kf, px, py, acc, bx, reinterpret_cast<const char *>(tile));
+            wg_barrier();
+            if (!todo) break;
+            l = ln;
+            h = hn;
+            lv = lvn;
+        }
+    }
+    if (active) {
+#pragma unroll
+        for (int it = 0; it < NI; ++it) voxel_store<KC>(out, a, i, j, k0, b + it, acc + it * KC);
+    }
 }
 
 // Cell gather of one workgroup with its z-prefix lookups served from LDS.  The 4 waves

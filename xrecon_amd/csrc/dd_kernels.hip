@@ -322,25 +322,34 @@ __global__ __launch_bounds__(kBlock, STAGE ? (R <= 8 ? 4 : 3) : 1) void k_cell(c
     else cell_body<OPK, GEO, R, 0, false>(hdr, lineC, colt, WX, WY, out, a, c, r0, v, b, wgrp);
 }
 
-// 32-slice chunks: at most 128 registers (4 waves per SIMD); uncapped they take 133 and
-// run at 3 waves, 24 % slower on the 512^2 x 256 cone-arc workload.
-template <int OPK, int GEO, int KC, bool HALVES>
-__global__ __launch_bounds__(kBlock, KC >= 32 ? 4 : 1) void k_voxel(const ViewHdr *__restrict__ hdr, const float4 *__restrict__ lineV,
-                                                  const float4 *__restrict__ colt, const VoxTile *__restrict__ vtile,
-                                                  const float2 *__restrict__ Q, float *__restrict__ out,
-                                                  float *__restrict__ part, VoxArgs a)
+// Waves per SIMD that the voxel gathers are compiled for: as many as their blocks leave
+// room for (vox_lds).  Pairs of items of B and B_W would spill 13 registers at 5.
+constexpr int vox_waves(int op, int KC, int NI, bool fit)
 {
-    __shared__ __attribute__((aligned(16))) float2 tile[vox_lds(KC)];
+    if (!fit) return KC * NI >= 32 ? 4 : 1;
+    if (NI == 1) return KC >= 32 ? 5 : 6;
+    return KC < 16 || op == VOX_AT ? 5 : 4;
+}
+
+// A workgroup sums NI batch items at once: the rows, columns and weights of a lookup are
+// the same for all items (4 of the 7 instructions of a lookup).
+template <int OPK, int GEO, int KC, int NI, bool FIT>
+__global__ __launch_bounds__(kBlock, vox_waves(OPK, KC, NI, FIT)) void k_voxel(const ViewHdr *__restrict__ hdr, const float4 *__restrict__ lineV,
+                                                  const float4 *__restrict__ colt, const float *__restrict__ cols,
+                                                  const VoxTile *__restrict__ vtile, const float2 *__restrict__ Q,
+                                                  float *__restrict__ out, float *__restrict__ part, VoxArgs a)
+{
+    __shared__ __attribute__((aligned(16))) float2 tile[NI * (FIT ? vox_lds(KC, NI) : vox_lds_rounds(KC, NI))];
     int i, j;
     voxel_coords(blockIdx.x, blockIdx.y, threadIdx.x, i, j);
     const int set = blockIdx.z % a.vsplit, rest = blockIdx.z / a.vsplit;
     const int chunk = rest % a.nchunk;
-    const int b = rest / a.nchunk;
+    const int b = a.b0 + NI * (rest / a.nchunk);
     const int v0 = set * a.vper, v1 = imin(a.nview, v0 + a.vper);
     // one view set: its own partial volume; no split: the output itself
     float *dst = a.vsplit > 1 ? part + (int64_t)set * a.nbatch * a.nz * a.ny * a.nx : out;
-    voxel_wg<OPK, GEO, KC, HALVES>(hdr, lineV, colt, vtile, Q, dst, a, i, j, i < a.nx && j < a.ny,
-                                   blockIdx.y * gridDim.x + blockIdx.x, chunk * KC, b, v0, v1, tile);
+    voxel_wg<OPK, GEO, KC, NI, FIT>(hdr, lineV, colt, cols, vtile, Q, dst, a, i, j, i < a.nx && j < a.ny,
+                               blockIdx.y * gridDim.x + blockIdx.x, chunk * KC, b, v0, v1, tile);
 }
 
 // out[e] = sum over sets s = 0..nset-1 of part[s * n + e], in set order.
@@ -436,19 +445,45 @@ void launch_cell(const Plan3d &p, int R, bool stage, const float2 *WX, const flo
                                           WX, WY, out, nbatch, s);
 }
 
+// nitem batch items from b0 on, NI at a time.
+template <int OPK, int GEO, int KC, int NI>
+void launch_voxel_items(const Plan3d &p, const float2 *Q, float *out, float *part, int nbatch, int b0, int nitem,
+                        hipStream_t s)
+{
+    VoxArgs a = make_vox_args(p, nbatch, KC);
+    a.b0 = b0;
+    const dim3 grid(ceil_div(a.nx, kVoxTile), ceil_div(a.ny, kVoxTile), nitem / NI * a.nchunk * a.vsplit);
+    if constexpr (KC >= kVoxStageMin) {
+        if (p.vox_fit & vox_fit_bit(KC, NI)) {
+            hipLaunchKernelGGL((k_voxel<OPK, GEO, KC, NI, true>), grid, dim3(kBlock), 0, s, p.d_hdr, p.d_lineV, p.d_col,
+                               p.d_cols, p.d_vtile, Q, out, part, a);
+            return;
+        }
+    }
+    if constexpr (NI == 1)
+        hipLaunchKernelGGL((k_voxel<OPK, GEO, KC, 1, false>), grid, dim3(kBlock), 0, s, p.d_hdr, p.d_lineV, p.d_col,
+                           p.d_cols, p.d_vtile, Q, out, part, a);
+}
+
+// Chunks of 8 and 16 slices: two items per workgroup (vox_pairs), an odd last one alone.
+template <int OPK, int GEO, int KC>
+void launch_voxel_pairs(const Plan3d &p, const float2 *Q, float *out, float *part, int nbatch, hipStream_t s)
+{
+    const int pairs = vox_pairs(p, KC, nbatch) ? nbatch & ~1 : 0;
+    if (pairs) launch_voxel_items<OPK, GEO, KC, 2>(p, Q, out, part, nbatch, 0, pairs, s);
+    if (nbatch > pairs) launch_voxel_items<OPK, GEO, KC, 1>(p, Q, out, part, nbatch, pairs, nbatch - pairs, s);
+}
+
 template <int OPK, int GEO>
 void launch_voxel(const Plan3d &p, int KC, const float2 *Q, float *out, float *part, int nbatch, hipStream_t s)
 {
-    const VoxArgs a = make_vox_args(p, nbatch, KC);
-    dim3 grid(ceil_div(a.nx, kVoxTile), ceil_div(a.ny, kVoxTile), nbatch * a.nchunk * a.vsplit);
-    switch (KC) {
-    case 1: hipLaunchKernelGGL((k_voxel<OPK, GEO, 1, false>), grid, dim3(kBlock), 0, s, p.d_hdr, p.d_lineV, p.d_col, p.d_vtile, Q, out, part, a); break;
-    case 4: hipLaunchKernelGGL((k_voxel<OPK, GEO, 4, false>), grid, dim3(kBlock), 0, s, p.d_hdr, p.d_lineV, p.d_col, p.d_vtile, Q, out, part, a); break;
-    case 8: hipLaunchKernelGGL((k_voxel<OPK, GEO, 8, false>), grid, dim3(kBlock), 0, s, p.d_hdr, p.d_lineV, p.d_col, p.d_vtile, Q, out, part, a); break;
-    case 16: hipLaunchKernelGGL((k_voxel<OPK, GEO, 16, false>), grid, dim3(kBlock), 0, s, p.d_hdr, p.d_lineV, p.d_col, p.d_vtile, Q, out, part, a); break;
-    case 16 | XR_VOXEL_HALVES: hipLaunchKernelGGL((k_voxel<OPK, GEO, 16, true>), grid, dim3(kBlock), 0, s, p.d_hdr, p.d_lineV, p.d_col, p.d_vtile, Q, out, part, a); break;
-    default:  // 32 | XR_VOXEL_HALVES: valid_chunk admits nothing else
-        hipLaunchKernelGGL((k_voxel<OPK, GEO, 32, true>), grid, dim3(kBlock), 0, s, p.d_hdr, p.d_lineV, p.d_col, p.d_vtile, Q, out, part, a); break;
+    switch (chunk_slices(KC)) {
+    case 1: launch_voxel_items<OPK, GEO, 1, 1>(p, Q, out, part, nbatch, 0, nbatch, s); break;
+    case 4: launch_voxel_items<OPK, GEO, 4, 1>(p, Q, out, part, nbatch, 0, nbatch, s); break;
+    case 8: launch_voxel_pairs<OPK, GEO, 8>(p, Q, out, part, nbatch, s); break;
+    case 16: launch_voxel_pairs<OPK, GEO, 16>(p, Q, out, part, nbatch, s); break;
+    default:  // 32: valid_chunk admits nothing else
+        launch_voxel_items<OPK, GEO, 32, 1>(p, Q, out, part, nbatch, 0, nbatch, s); break;
     }
 }
 
@@ -549,7 +584,7 @@ int execute_fdk(const Plan3d &p, const float *in, float *out, int nbatch, const 
     const size_t need = workspace_bytes(p, XR_OP_BACKPROJECTION_W, nbatch);
     if (ws_bytes < need || !ws)
         return fail(XR_EWORKSPACE, "workspace of " + std::to_string(ws_bytes) + " bytes, need " + std::to_string(need));
-    if (voxel_chunk == 0) voxel_chunk = default_chunk(p);
+    if (voxel_chunk == 0) voxel_chunk = default_chunk(p, nbatch);
     if (!valid_chunk(voxel_chunk)) return fail(XR_EINVAL, "voxel_chunk must be 1, 4, 8, 16, 16 | XR_VOXEL_HALVES or 32 | XR_VOXEL_HALVES");
     float2 *Q = static_cast<float2 *>(ws);
     // the taps live where the view-split partial volumes go later (workspace_bytes
@@ -633,7 +668,7 @@ int execute_phase(const Plan3d &p, int op, int phase, const float *in, float *ou
     const int cell_mode = tile_rows & (XR_CELL_DIRECT | XR_CELL_LDS);
     tile_rows &= ~(XR_CELL_DIRECT | XR_CELL_LDS);
     if (tile_rows == 0) tile_rows = default_rows(p);
-    if (voxel_chunk == 0) voxel_chunk = default_chunk(p);
+    if (voxel_chunk == 0) voxel_chunk = default_chunk(p, nbatch);
     if (!valid_rows(tile_rows) || cell_mode == (XR_CELL_DIRECT | XR_CELL_LDS))
         return fail(XR_EINVAL, "tile_rows must be 1, 2, 4, 8 or 16, with at most one of XR_CELL_DIRECT, XR_CELL_LDS");
     const bool stage = cell_mode == XR_CELL_LDS || (cell_mode == 0 && make_cell_args(p, 1).band);

@@ -11,7 +11,7 @@
 #include <cmath>
 #include <cstring>
 
-#include "slice.h"
+#include "dd_body.h"
 
 namespace xr {
 
@@ -89,6 +89,7 @@ int build_tables(Plan3d &p, const float *angles, PlanTables &t, std::string &err
     t.lineC.assign((size_t)V * ML, float4{0, 0, 0, 0});
     t.lineV.assign((size_t)V * ML, float4{0, 0, 0, 0});
     t.col.assign((size_t)V * (nu + 1), float4{0, 0, 0, 0});
+    t.cols.assign((size_t)V * 3 * (nu + kColPad), 0.0f);
     p.xdrv.assign(V, 0);
     p.keep.assign(V, 0);
     p.any_x = p.any_y = 0;
@@ -218,8 +219,13 @@ int build_tables(Plan3d &p, const float *angles, PlanTables &t, std::string &err
             t.col[cb0 + c] = float4{(float)d[c], (float)sig[c], (float)(1.0 / (sig[c] * dvv)),
                                     (float)(cone ? d[c + 1] - d[c] : du)};
         t.col[cb0 + nu] = float4{(float)d[nu], 0.0f, 0.0f, 0.0f};
-        if (is_slice(p))
-            for (int c = 0; c < nu + kSlicePad; ++c) t.dcol.push_back((float)d[std::min(c, nu)]);
+        float *cols = t.cols.data() + (size_t)v * 3 * (nu + kColPad);
+        for (int c = 0; c < nu + kColPad; ++c) {
+            const float4 &e = t.col[cb0 + std::min(c, nu)];
+            cols[c] = e.x;
+            cols[nu + kColPad + c] = e.z;
+            cols[2 * (nu + kColPad) + c] = e.y;
+        }
         h.dlo = (float)d[0];
         h.dhi = (float)d[nu];
         // Span class: the widest column, measured in pixel widths of the line with the
@@ -270,13 +276,7 @@ int build_tables(Plan3d &p, const float *angles, PlanTables &t, std::string &err
         }
     }
 
-    // Voxel gathers on volumes too small to fill the GPU split their views into sets.
     const int gx = ceil_div(nx, kVoxTile), gy = ceil_div(ny, kVoxTile);
-    {
-        const int64_t groups = (int64_t)gx * gy * ceil_div(nz, chunk_slices(default_chunk(p)));
-        int sp = groups >= kVoxMinGroups ? 1 : (int)std::min<int64_t>(16, ceil_div(kVoxMinGroups, groups));
-        p.vsplit = std::max(1, std::min(sp, V));
-    }
 
     // Cell-gather column groups: depth-scale range of each group's columns per view, and
     // the span class from above.
@@ -394,6 +394,23 @@ int build_tables(Plan3d &p, const float *angles, PlanTables &t, std::string &err
                 else if (p.kind == GEO_ARC) vt = voxel_tile<GEO_ARC>(t.hdr[v], t.lineV.data(), ct, ny, nu, ML, v, i0, i1, j0, j1);
                 else vt = voxel_tile<GEO_PAR>(t.hdr[v], t.lineV.data(), ct, ny, nu, ML, v, i0, i1, j0, j1);
             }
+    }
+    const VoxArgs va = make_vox_args(p, 1, 1);
+    int misses = 0;
+    for (const VoxTile &vt : t.vtile) {
+        if (!(misses & 1) && !voxel_tile_fits<8, 1>(vt, va)) misses |= vox_fit_bit(8, 1);
+        if (!(misses & 2) && !voxel_tile_fits<16, 1>(vt, va)) misses |= vox_fit_bit(16, 1);
+        if (!(misses & 4) && !voxel_tile_fits<32, 1>(vt, va)) misses |= vox_fit_bit(32, 1);
+        if (!(misses & 8) && !voxel_tile_fits<8, 2>(vt, va)) misses |= vox_fit_bit(8, 2);
+        if (!(misses & 16) && !voxel_tile_fits<16, 2>(vt, va)) misses |= vox_fit_bit(16, 2);
+    }
+    p.vox_fit = 31 & ~misses;
+
+    // Voxel gathers on volumes too small to fill the GPU split their views into sets.
+    {
+        const int64_t groups = (int64_t)gx * gy * ceil_div(nz, nz >= 128 ? 32 : nz >= 64 ? 16 : nz >= 8 ? 8 : nz >= 4 ? 4 : 1);
+        int sp = groups >= kVoxMinGroups ? 1 : (int)std::min<int64_t>(16, ceil_div(kVoxMinGroups, groups));
+        p.vsplit = std::max(1, std::min(sp, V));
     }
     return XR_OK;
 }

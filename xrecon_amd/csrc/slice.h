@@ -27,14 +27,14 @@
 
 namespace xr {
 
-constexpr int kSlicePad = 4;     // zeros after each line of the tables
+constexpr int kSlicePad = kColPad;  // zeros after each line of the tables
 constexpr int kSliceSegs = 8;    // cell gather: waves per workgroup, each a run of the lines
 constexpr int kSliceUnroll = 4;  // ... and lines in flight per wave
 
 struct SliceArgs {
     const ViewHdr *hdr;
     const float4 *lineC, *lineV, *col;
-    const float *dcol;  // Plan3d::d_dcol
+    const float *cols;  // Plan3d::d_cols
     const CellGroup *cgrp;
     const int *citems;
     int nx, ny, nu, nview, maxline, nb;
@@ -70,7 +70,7 @@ inline int slice_waves(const Plan3d &p) { return ceil_div(p.vol.nx, 8) * ceil_di
 inline SliceArgs make_slice_args(const Plan3d &p, int nb)
 {
     SliceArgs a;
-    a.hdr = p.d_hdr; a.lineC = p.d_lineC; a.lineV = p.d_lineV; a.col = p.d_col; a.dcol = p.d_dcol;
+    a.hdr = p.d_hdr; a.lineC = p.d_lineC; a.lineV = p.d_lineV; a.col = p.d_col; a.cols = p.d_cols;
     a.cgrp = p.d_cgrp; a.citems = p.d_citems;
     a.nx = p.vol.nx; a.ny = p.vol.ny; a.nu = p.geo.nu; a.nview = p.nview; a.maxline = p.maxline; a.nb = nb;
     a.bg = slice_items(nb); a.ng = ceil_div(nb, a.bg);
@@ -115,26 +115,6 @@ void slice_run_many(SlicePass pass, int kind, int kop, int bg, int waves, const 
                     const SliceLaunch &l, hipStream_t s);
 
 #if defined(__HIPCC__)
-
-// N consecutive floats from a 4-byte aligned place, as one load.
-template <int N>
-__device__ inline void slice_load(const char *base, unsigned off, float *dst)
-{
-#if defined(__HIP_DEVICE_COMPILE__)
-    typedef float vec __attribute__((ext_vector_type(N), aligned(4)));
-    const vec r = *(const __attribute__((address_space(1))) vec *)((const __attribute__((address_space(1))) char *)base + off);
-#pragma unroll
-    for (int i = 0; i < N; ++i) dst[i] = r[i];
-#endif
-}
-
-// 1 / y to within an ulp: v_rcp_f32 and one Newton step (a division compiles to ten
-// instructions).
-__device__ inline float slice_rcp(float y)
-{
-    const float r = __builtin_amdgcn_rcpf(y);
-    return fmaf(fmaf(-y, r, 1.0f), r, r);
-}
 
 // w x, zero where w is zero, whatever x holds: one v_mul_legacy_f32.
 __device__ inline float mul_or_zero(float w, float x)
@@ -238,10 +218,10 @@ struct SliceWeight {
         if (GEO == GEO_PAR) return 1.0f;
         if (GEO == GEO_FLAT) {
             const float t = fmaf(q, u1, u0);
-            return slice_rcp(t * t);
+            return near_rcp(t * t);
         }
         const float e = u1 - q;
-        return slice_rcp(fmaf(e, e, u0));
+        return near_rcp(fmaf(e, e, u0));
     }
 };
 
@@ -273,10 +253,10 @@ __device__ inline void slice_lines(const SliceArgs &a, const ViewHdr &h, const f
         }
         const char *line = T + (int64_t)Lu * pitch;
         if (BG == 1) {
-            slice_load<NP>(line, m * 4u, f[u]);
+            load_floats<NP>(line, m * 4u, f[u]);
         } else {
 #pragma unroll
-            for (int q = 0; q < NP; ++q) slice_load<BG>(line, m * (BG * 4u) + q * (BG * 4u), f[u] + q * BG);
+            for (int q = 0; q < NP; ++q) load_floats<BG>(line, m * (BG * 4u) + q * (BG * 4u), f[u] + q * BG);
         }
         if (OPK == CELL_BWT) {
             const float dal = h.xdrv ? a.dx : a.dy, p0 = (0.5f - 0.5f * fal) * dal + (h.xdrv ? a.shx : a.shy);
@@ -318,7 +298,7 @@ __device__ inline void slice_line_any(const SliceArgs &a, const ViewHdr &h, cons
         float w = minf_finite(hi, m + 1.0f) - maxf_finite(lo, m);
         if (OPK == CELL_BWT) w *= U1.at(fmaf(m, dal, p0));
         float f[BG];
-        slice_load<BG>(line, (unsigned)m * (BG * 4u), f);
+        load_floats<BG>(line, (unsigned)m * (BG * 4u), f);
 #pragma unroll
         for (int b = 0; b < BG; ++b) s[b] = fmaf(w, f[b], s[b]);
     }
@@ -385,18 +365,6 @@ __device__ inline void slice_cell(const SliceArgs &a, int bid, const float *__re
     out[((int64_t)(g * BG + wave) * a.nview + v) * a.nu + (h.keep ? c : a.nu - 1 - c)] = s * q;
 }
 
-// atan(t) for the column seeds, which are corrected against the table: a least-squares odd
-// polynomial for |t| <= 0.6 (within 3e-7 rad; fans of up to 62 degrees), atanf beyond.
-__device__ inline float slice_atan(float t)
-{
-    if (wave_any(fabsf(t) > 0.6f)) return atanf(t);
-    const float q = t * t;
-    float r = fmaf(q, 0.0563796f, -0.1275247f);
-    r = fmaf(q, r, 0.1980930f);
-    r = fmaf(q, r, -0.3332516f);
-    return fmaf(t * q, r, t);
-}
-
 // One view of the voxel gather: the overlaps of the pixel's footprint [a0, a1] with three
 // columns at a time, from the one that the closed-form inverse gives (corrected where it
 // came out past the footprint's start; columns before it have no width).  XD: x-driven.
@@ -409,15 +377,15 @@ __device__ inline void slice_view(const SliceArgs &a, const ViewHdr &h, const fl
     const float e = fmaf(fm, lv.y, lv.x);
     const float a0 = clampf(e, h.dlo, h.dhi), a1 = clampf(e + lv.y, h.dlo, h.dhi);
     const float T = seed_div(fmaf(h.tp1, a0, h.tp0), fmaf(h.tq1, a0, h.tq0));
-    int c = (int)clampf(fmaf(h.tk1, GEO == GEO_ARC ? slice_atan(T) : T, h.tk0), 0.0f, (float)(a.nu - 1));
+    int c = (int)clampf(fmaf(h.tk1, GEO == GEO_ARC ? seed_atan(T) : T, h.tk0), 0.0f, (float)(a.nu - 1));
     float d[4], s[3 * BG];
     auto load = [&]() {
-        slice_load<4>(dt, (unsigned)c * 4u, d);
+        load_floats<4>(dt, (unsigned)c * 4u, d);
         if (BG == 1) {
-            slice_load<3>(st, (unsigned)c * 4u, s);
+            load_floats<3>(st, (unsigned)c * 4u, s);
         } else {
 #pragma unroll
-            for (int q = 0; q < 3; ++q) slice_load<BG>(st, (unsigned)c * (BG * 4u) + q * (BG * 4u), s + q * BG);
+            for (int q = 0; q < 3; ++q) load_floats<BG>(st, (unsigned)c * (BG * 4u) + q * (BG * 4u), s + q * BG);
         }
     };
     load();
@@ -439,8 +407,8 @@ __device__ inline void slice_view(const SliceArgs &a, const ViewHdr &h, const fl
     if (wave_any(d[3] < a1)) {  // pixels over more than three columns
         for (int k = c + 3; k < a.nu && b0 < a1; ++k) {
             float dn, x[BG];
-            slice_load<1>(dt, (unsigned)(k + 1) * 4u, &dn);
-            slice_load<BG>(st, (unsigned)k * (BG * 4u), x);
+            load_floats<1>(dt, (unsigned)(k + 1) * 4u, &dn);
+            load_floats<BG>(st, (unsigned)k * (BG * 4u), x);
             const float b1 = clampf(dn, a0, a1);
 #pragma unroll
             for (int b = 0; b < BG; ++b) sum[b] += mul_or_zero(b1 - b0, x[b]);
@@ -490,7 +458,7 @@ __device__ inline void slice_voxel(const SliceArgs &a, int bid, const float *__r
         const int vn = imin(v + NW, a.nview - 1);
         hn = ro_load(a.hdr + vn);
         ln = line_of(vn, hn);
-        const float *dt = a.dcol + (int64_t)v * sp, *st = Sg + (int64_t)v * sp * BG;
+        const float *dt = a.cols + (int64_t)v * 3 * sp, *st = Sg + (int64_t)v * sp * BG;
         if (wave_uniform(h.xdrv)) slice_view<OPK, GEO, BG, true>(a, h, lv, dt, st, fx, ppx, ppy, acc);
         else slice_view<OPK, GEO, BG, false>(a, h, lv, dt, st, fy, ppy, ppx, acc);
     }

@@ -94,6 +94,7 @@ struct Plan3d {
     int maxline = 0;         // max(Nx, Ny)
     int any_x = 0, any_y = 0;
     int big = 0;             // z-prefix table of one batch item >= 2^32 bytes or plane >= 2^24 bytes
+    int vox_fit = 0;         // vox_fit_bit(KC, NI) set: every block of the voxel gather fits the LDS then
     int vsplit = 1;          // voxel gathers: views split over this many workgroup sets (summed after)
     // Scalars shared by all views.
     float zb = 0, dz = 1;    // volume bottom z and slice thickness
@@ -109,7 +110,7 @@ struct Plan3d {
     float4 *d_lineC = nullptr;  // [nview][maxline] {toff, invd, iz, lam}: cell kernels
     float4 *d_lineV = nullptr;  // [nview][maxline] {P0, Delta, zeta, 1/(Delta zeta)}: voxel kernels
     float4 *d_col = nullptr;    // [nview][Nu+1]    {d, sigma, kappa, W}
-    float *d_dcol = nullptr;    // 2D: [nview][Nu+4] the column boundaries d alone (d_Nu repeated at the end)
+    float *d_cols = nullptr;    // [nview][3][Nu+4]: d (d_Nu repeated at the end), kappa, sigma of d_col
     VoxTile *d_vtile = nullptr; // [nview][ceil(Ny/16)][ceil(Nx/16)]: voxel-gather staging estimates
     CellGroup *d_cgrp = nullptr; // [nview][ceil(Nu/64)]: cell-gather column groups
     int *d_citems = nullptr;     // the groups v * ceil(Nu/64) + g listed by span class (2, then 3, then 0),
@@ -127,7 +128,7 @@ struct Plan3d {
 struct PlanTables {
     std::vector<ViewHdr> hdr;
     std::vector<float4> lineC, lineV, col;
-    std::vector<float> dcol;
+    std::vector<float> cols;  // as Plan3d::d_cols
     std::vector<VoxTile> vtile;
     std::vector<CellGroup> cgrp;
     std::vector<int> citems;  // as Plan3d::d_citems
