@@ -17,6 +17,7 @@
 #include <string>
 #include <vector>
 
+#include "column.h"
 #include "slice.h"
 
 namespace xr {
@@ -35,7 +36,8 @@ struct BatchDesc {
     VoxArgs va;  // nchunk is filled per launch from the launch's voxel chunk
     SinoArgs sa;
     int nb, any_y;
-    int big;  // Plan3d::big
+    int big;   // Plan3d::big
+    int cell;  // 1: the cell gathers use the z-prefix tables
     unsigned long long ws_volx, ws_voly, ws_sino;  // byte offsets into the workspace
     unsigned long long ws_part;                    // view-set partial volumes (va.vsplit > 1)
 };
@@ -48,11 +50,11 @@ struct IOPtrs {
 // Block counts per instance and pass (identical on host and device).
 __host__ __device__ inline int blocks_vol_prefix(const BatchDesc &d)
 {
-    return ceil_div((int64_t)d.nb * d.ca.nx * d.ca.ny, kBlock);
+    return d.cell ? ceil_div((int64_t)d.nb * d.ca.nx * d.ca.ny, kBlock) : 0;
 }
 __host__ __device__ inline int blocks_transpose(const BatchDesc &d)
 {
-    return d.any_y ? ceil_div(d.ca.nx, 32) * ceil_div(d.ca.ny, 32) * d.nb * (d.ca.nz + 1) : 0;
+    return d.cell && d.any_y ? ceil_div(d.ca.nx, 32) * ceil_div(d.ca.ny, 32) * d.nb * (d.ca.nz + 1) : 0;
 }
 // Column groups of span-class index K (0: two-pixel, 1: three-pixel, 2: general, 3: all).
 __host__ __device__ inline int cell_class_items(const BatchDesc &d, int K)
@@ -66,7 +68,7 @@ __host__ __device__ inline int cell_class_offset(const BatchDesc &d, int K)
 // Workgroups of class index K at R rows: quads of groups x row tiles x batch items.
 __host__ __device__ inline int blocks_cell(const BatchDesc &d, int R, int K)
 {
-    return ceil_div(cell_class_items(d, K), kWavesPerBlock) * ceil_div(d.ca.nv, R) * d.nb;
+    return d.cell ? ceil_div(cell_class_items(d, K), kWavesPerBlock) * ceil_div(d.ca.nv, R) * d.nb : 0;
 }
 // Rows per thread of span-class index K: R for the two-pixel class, at most 8 otherwise.
 __host__ __device__ inline int cell_class_rows(int R, int K) { return K == 0 || R <= 8 ? R : 8; }
@@ -376,6 +378,9 @@ struct xr_batch3d {
     std::vector<xr::SliceArgs> slices;
     std::vector<size_t> off_cell, off_vox;
     xr::SliceArgs *d_slices = nullptr;
+    // plans whose cell gathers take the two steps of column.h (rows = 0: the others)
+    std::vector<xr::ColArgs> cols;
+    xr::ColArgs *d_cols = nullptr;
     int device = 0;
     size_t ws_cell = 0, ws_vox = 0;
 };
@@ -409,6 +414,35 @@ int run_slice_pass(const xr_batch3d &b, xr::SlicePass pass, const xr::Route &rt,
             if (total > 0)
                 xr::slice_run_many(pass, b.plans[0]->kind, rt.kop, bg, waves, b.d_slices, n, l, s);
         }
+    return XR_OK;
+}
+
+// One pass of the two-step cell gathers of a batch: a launch for the plans that split their
+// lines and one for those that do not.
+int run_col_pass(const xr_batch3d &b, xr::ColPass pass, const xr::Route &rt, const xr::IOPtrs &io, char *ws,
+                 hipStream_t s)
+{
+    const int n = (int)b.cols.size();
+    xr::ColLaunch l{};
+    for (int split = 0; split < (pass == xr::COL_TABLES ? 1 : 2); ++split) {
+        int64_t total = 0;
+        size_t lds = 0;
+        for (int i = 0; i < n; ++i) {
+            const xr::ColArgs &a = b.cols[i];
+            l.start[i] = (int)total;
+            if (a.rows > 0 && (pass == xr::COL_TABLES || a.split == split)) {
+                total += xr::col_pass_blocks(pass, a);
+                lds = std::max(lds, xr::col_lds_bytes(a));
+                l.in[i] = io.in[i];
+                l.out[i] = io.out[i];
+                l.t0[i] = reinterpret_cast<float *>(ws + b.desc[i].ws_volx);
+                l.t1[i] = xr::col_second_table(*b.plans[i], l.t0[i], a.nb);
+            }
+            if (total >= INT32_MAX) return fail(XR_EINVAL, "batch too large for one launch");
+        }
+        l.start[n] = (int)total;
+        if (total > 0) xr::col_run_many(pass, b.plans[0]->kind, rt.kop, split, lds, b.d_cols, n, l, s);
+    }
     return XR_OK;
 }
 
@@ -466,12 +500,14 @@ int xr_batch3d_create(xr_plan3d *const *plans, int n, const int *num_batch, xr_b
         const size_t vb = xr::align256(xr::vol_prefix_bytes(p, num_batch[i]));
         d.ws_volx = off_cell;
         d.ws_voly = off_cell + vb;
-        off_cell += vb * (p.any_y ? 2 : 1);
+        off_cell += std::max(vb * (p.any_y ? 2 : 1), xr::col_table_bytes(p, num_batch[i]));
         d.ws_sino = off_vox;
         off_vox += xr::align256(xr::sino_prefix_bytes(p, num_batch[i]));
         d.ws_part = off_vox;
         off_vox += xr::align256(xr::split_partial_bytes(p, num_batch[i]));
+        d.cell = p.col_rows == 0;
         b->desc.push_back(d);
+        b->cols.push_back(xr::make_col_args(p, num_batch[i]));
         b->plans.push_back(&p);
     }
     b->ws_cell = off_cell;
@@ -485,8 +521,14 @@ int xr_batch3d_create(xr_plan3d *const *plans, int n, const int *num_batch, xr_b
     const void *src = b->slice ? (const void *)b->slices.data() : (const void *)b->desc.data();
     hipError_t e = hipMalloc(dst, bytes);
     if (e == hipSuccess) e = hipMemcpy(*dst, src, bytes, hipMemcpyHostToDevice);
+    if (!b->slice) {
+        const size_t cb = sizeof(xr::ColArgs) * n;
+        if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void **>(&b->d_cols), cb);
+        if (e == hipSuccess) e = hipMemcpy(b->d_cols, b->cols.data(), cb, hipMemcpyHostToDevice);
+    }
     if (prev >= 0 && prev != b->device) (void)hipSetDevice(prev);
     if (e != hipSuccess) {
+        if (b->d_cols) (void)hipFree(b->d_cols);
         if (*dst) (void)hipFree(*dst);
         return fail(XR_ENOMEM, std::string("batch descriptor upload failed: ") + hipGetErrorString(e));
     }
@@ -499,6 +541,7 @@ void xr_batch3d_destroy(xr_batch3d *b)
     if (!b) return;
     if (b->d_desc) (void)hipFree(b->d_desc);
     if (b->d_slices) (void)hipFree(b->d_slices);
+    if (b->d_cols) (void)hipFree(b->d_cols);
     delete b;
 }
 
@@ -598,7 +641,11 @@ int xr_batch3d_execute(const xr_batch3d *b, int op, const float *const *in, floa
             const int rows = k == 3 ? R : xr::cell_class_rows(R, k);
             gs[k] = xr::block_starts(b->desc, [rows, k](const BatchDesc &d) { return xr::blocks_cell(d, rows, k); });
         }
-        hipLaunchKernelGGL(xr::k_vol_prefix_batch, dim3((int)g_pre), dim3(xr::kBlock), 0, s, D, n, pre, io, ws);
+        int rc = run_col_pass(*b, xr::COL_TABLES, rt, io, ws, s);
+        if (!rc) rc = run_col_pass(*b, xr::COL_GATHER, rt, io, ws, s);
+        if (rc) return rc;
+        if (g_pre > 0)
+            hipLaunchKernelGGL(xr::k_vol_prefix_batch, dim3((int)g_pre), dim3(xr::kBlock), 0, s, D, n, pre, io, ws);
         if (g_tr > 0)
             hipLaunchKernelGGL(xr::k_transpose_batch, dim3((int)g_tr), dim3(xr::kBlock), 0, s, D, n, tr, ws);
     } else {

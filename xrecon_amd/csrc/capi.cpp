@@ -8,7 +8,7 @@
 #include <memory>
 #include <string>
 
-#include "xr_internal.h"
+#include "column.h"
 
 namespace xr {
 const char *last_error();
@@ -146,6 +146,7 @@ int xr_plan3d_create(const xr_volume3d *vol, const xr_geometry3d *geo, const flo
     std::string err;
     rc = xr::build_tables(p, angles_host, t, err);
     if (rc) return fail(rc, err);
+    xr::column_plan(p, t);
     DeviceGuard g(device);
     if ((rc = upload(&p.d_hdr, t.hdr)) || (rc = upload(&p.d_lineC, t.lineC)) || (rc = upload(&p.d_lineV, t.lineV)) ||
         (rc = upload(&p.d_col, t.col)) || (rc = upload(&p.d_cols, t.cols)) || (rc = upload(&p.d_vtile, t.vtile)) ||

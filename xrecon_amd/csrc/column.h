@@ -1,0 +1,422 @@
+// Cell gathers (A, B^T, B_W^T) that resample a line in two steps, first along the detector
+// columns, then along the rows.
+//
+// A lane owns one detector column and a tile of up to 16 rows of one view.  On each line it
+// first sums the pixels that its column overlaps, slice by slice over the few slices that
+// its rows reach, and keeps the running sums in LDS entries of its own (no other lane reads
+// them: no barrier); then each row boundary is one lookup there, whatever the number of
+// pixels.  The gathers over z-prefix tables (dd_kernels.hip) look up every pixel at every
+// row boundary instead: 13 instructions per row with two pixels and 22 with three, against
+// 7 here and as many per slice as there are pixels.
+//
+// The volume is read from plain copies in both line orientations: slices in planes,
+// kColPad zeros after each line, and at least one zero slice after the last, so that slices
+// come in pairs.  The running sums start at the tile's first slice, so they stay within the
+// tile's own depth (no cancellation against the whole column's sum).  The copies take 0.28 ms
+// for 512^2 x 256 where the prefix tables took 0.76.
+//
+// Bound by VALU issue (95 % busy on 256^2 x 64, 720 views of 512 x 64; about 200 instructions
+// per line and wave, of which 112 are the 16 rows', 25 the slices').  A plan takes this path
+// (Plan3d::col_rows > 0) when its tiles' slices fit the LDS (column_plan).  The z-prefix
+// gathers remain for rows of more than 9 slices and for volumes beyond 24-bit planes or
+// 32-bit offsets.  Whole call before and after: 256^2 x 64, 720 views of 512 x 64 flat 2.84
+// and 2.00 ms; 256^2 x 10, 360 views of 256 x 10 0.34 and 0.23 ms; 512^2 x 256, 1152 views of
+// 736 x 128 arc 30.6 and 20.1 ms.
+#pragma once
+
+#include <type_traits>
+
+#include "dd_body.h"
+
+namespace xr {
+
+constexpr int kColSlices = 2;   // slices come in pairs
+constexpr int kColMax = 40;     // most slices of a tile
+constexpr int kColRows = 16;    // most rows of a tile
+// Slices that a tile of more than 4 rows may take: the LDS of 20 waves per CU, which is what
+// the registers allow.  512^2 x 256 on 736 x 128, 1152 views: 16 rows with 36 slices 24.1 ms,
+// 8 rows with 20 slices 25.5 ms (4 rows 44.5 ms with 12), 16 rows with 22 slices 19.7 ms.
+constexpr int kColFit = 30;
+// Fewer waves than this (an MI355X holds 5120) split their lines over four: 1440 waves
+// (256^2 x 10, 360 views) take 0.24 ms split and 0.42 unsplit, 7218 take 1.14 and 1.13, 8640
+// 1.16 and 1.19, 23040 2.14 and 2.13.
+constexpr int64_t kColSplitMax = 8192;
+
+struct ColArgs {
+    const ViewHdr *hdr;
+    const float4 *lineC, *col;
+    const CellGroup *cgrp;
+    const int *citems;
+    int nx, ny, nz, nu, nv, nview, maxline, nb;
+    int nzp;                 // slices of the tables
+    int rows, ntile;         // rows per tile, tiles
+    int ns;                  // LDS slices per lane
+    int nitems, ncg;         // column groups over all views, per view
+    int any_y, split;  // split: the 4 waves of a workgroup share one item's lines, else it is one wave
+    float v0, dvv, vc, zoff, sod, dx, dy, shx, shy;
+};
+
+inline int col_slices(int nz) { return (nz + 1 + kColSlices - 1) / kColSlices * kColSlices; }
+
+inline int64_t col_table_floats(const Plan3d &p, int nb, bool ydrv)
+{
+    return (int64_t)nb * col_slices(p.vol.nz) *
+           (ydrv ? (int64_t)p.vol.nx * (p.vol.ny + kColPad) : (int64_t)p.vol.ny * (p.vol.nx + kColPad));
+}
+inline size_t col_table_bytes(const Plan3d &p, int nb)
+{
+    return align256((size_t)col_table_floats(p, nb, false) * sizeof(float)) +
+           (p.any_y ? align256((size_t)col_table_floats(p, nb, true) * sizeof(float)) : 0);
+}
+
+inline ColArgs make_col_args(const Plan3d &p, int nb)
+{
+    ColArgs a;
+    a.hdr = p.d_hdr; a.lineC = p.d_lineC; a.col = p.d_col; a.cgrp = p.d_cgrp; a.citems = p.d_citems;
+    a.nx = p.vol.nx; a.ny = p.vol.ny; a.nz = p.vol.nz; a.nu = p.geo.nu; a.nv = p.geo.nv;
+    a.nview = p.nview; a.maxline = p.maxline; a.nb = nb;
+    a.nzp = col_slices(a.nz);
+    a.rows = p.col_rows; a.ntile = ceil_div(a.nv, imax(a.rows, 1)); a.ns = p.col_ns;
+    a.ncg = ceil_div(a.nu, kWave); a.nitems = a.ncg * a.nview;
+    a.any_y = p.any_y; a.split = p.col_split;
+    a.v0 = p.v0; a.dvv = p.dvv; a.vc = (float)((double)p.v0 + 0.5 * a.nv * (double)p.dvv);
+    a.zoff = p.zoff; a.sod = p.sod;
+    a.dx = p.vol.dx; a.dy = p.vol.dy; a.shx = p.vol.shift_x; a.shy = p.vol.shift_y;
+    return a;
+}
+
+__host__ __device__ inline int64_t col_table_blocks(const ColArgs &a)
+{
+    return (int64_t)ceil_div(a.nx + kColPad, 32) * ceil_div(a.ny + kColPad, 32) * a.nzp * a.nb;
+}
+__host__ __device__ inline int64_t col_blocks(const ColArgs &a)
+{
+    return (int64_t)a.nitems * a.ntile * a.nb;
+}
+__host__ __device__ inline size_t col_lds_bytes(const ColArgs &a)
+{
+    // (the split sum of 16 rows also goes through it)
+    return (size_t)(a.split ? kWavesPerBlock * imax(a.ns + 1, kColRows) : a.ns + 1) * kWave * sizeof(float);
+}
+
+// Slices a lane needs on a line where a row is `step` slices tall: its rows' height, the
+// two it starts and ends in, in whole loads.  step: an upper bound over the lanes.
+__host__ __device__ inline int col_line_slices(float step, int rows, int nzp)
+{
+    const int n = (int)(step * (float)rows * 1.0001f + 0.01f) + 2;
+    return imin((n + kColSlices - 1) / kColSlices * kColSlices, nzp);
+}
+
+enum ColPass : int { COL_TABLES, COL_GATHER };
+
+// One launch over several instances: first block, buffers and tables of each.
+struct ColLaunch {
+    int start[XR_BATCH_MAX + 1];
+    const float *in[XR_BATCH_MAX];
+    float *out[XR_BATCH_MAX], *t0[XR_BATCH_MAX], *t1[XR_BATCH_MAX];
+};
+
+// column_kernels.hip
+void column_plan(Plan3d &p, const PlanTables &t);
+int64_t col_pass_blocks(ColPass pass, const ColArgs &a);
+float *col_second_table(const Plan3d &p, void *ws, int nb);
+int col_run(const Plan3d &p, ColPass pass, int kop, const float *in, float *out, int nb, void *ws, hipStream_t s);
+void col_run_many(ColPass pass, int kind, int kop, bool split, size_t lds, const ColArgs *args, int n,
+                  const ColLaunch &l, hipStream_t s);
+
+#if defined(__HIPCC__)
+
+// TX[b][k][j][i], TY[b][k][i][Ny-1-j]: one 32 x 32 tile of one slice.
+__device__ inline void col_tables(const ColArgs &a, int bid, const float *__restrict__ f, float *__restrict__ TX,
+                                  float *__restrict__ TY)
+{
+    __shared__ float tile[32][33];
+    const int px = a.nx + kColPad, py = a.ny + kColPad;
+    const int tx = ceil_div(px, 32), ty = ceil_div(py, 32);
+    const int i0 = bid % tx * 32, j0 = bid / tx % ty * 32, q = bid / (tx * ty), b = q / a.nzp, k = q - b * a.nzp;
+    const int l = threadIdx.x & 31, r0 = threadIdx.x >> 5;
+    const float *src = f + ((int64_t)b * a.nz + k) * a.ny * a.nx;
+    for (int r = r0; r < 32; r += 8) {
+        const int i = i0 + l, j = j0 + r;
+        const float x = k < a.nz && i < a.nx && j < a.ny ? src[(int64_t)j * a.nx + i] : 0.0f;
+        tile[r][l] = x;
+        if (i < px && j < a.ny) TX[((int64_t)q * a.ny + j) * px + i] = x;
+    }
+    if (!a.any_y) return;
+    __syncthreads();
+    for (int r = r0; r < 32; r += 8) {
+        const int i = i0 + r, j = j0 + l;
+        if (i < a.nx && j < py) TY[((int64_t)q * a.nx + i) * py + (j < a.ny ? a.ny - 1 - j : j)] = tile[l][r];
+    }
+}
+
+__device__ inline void lds_store(char *base, unsigned off, float x)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    *(__attribute__((address_space(3))) float *)((__attribute__((address_space(3))) char *)base + off) = x;
+#endif
+}
+
+// Byte address of entry (int)z of a lane's block, z in [0, 256): the index goes straight into
+// byte 1 of the lane's address, whose byte 0 stays and whose upper bytes are zero.
+__device__ inline void entry_address(unsigned &addr, float z)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm("v_cvt_u32_f32_sdwa %0, %1 dst_sel:BYTE_1 dst_unused:UNUSED_PRESERVE src0_sel:DWORD" : "+v"(addr) : "v"(z));
+#endif
+}
+
+// The entry at an LDS address and the one a slice up.
+__device__ inline void lds_entries(unsigned addr, float &lo, float &hi)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    typedef __attribute__((address_space(3))) const float *lds_ptr;
+    const lds_ptr q = (lds_ptr)addr;
+    lo = q[0];
+    hi = q[kWave];
+#endif
+}
+
+// The LDS address of p, as a number.
+__device__ inline unsigned lds_address(char *p)
+{
+    unsigned a = 0;
+#if defined(__HIP_DEVICE_COMPILE__)
+    a = (unsigned)(__attribute__((address_space(3))) char *)p;
+    asm volatile("" : "+v"(a)::"memory");
+#endif
+    return a;
+}
+
+// N slices of a line from slice k0 of the lane's: its running sum goes on over NP pixels
+// with weights w, entry k the sum of the slices below k.
+template <int NP, int N>
+__device__ inline void col_slices(const char *line, unsigned off, int64_t plane, const float *w, int k0, char *mine,
+                                  float &run)
+{
+    float f[N][NP];
+    asm volatile("" : "+v"(off));  // (an address per group: base in SGPRs, this offset)
+#pragma unroll
+    for (int i = 0; i < N; ++i) load_floats<NP>(line + (k0 + i) * plane, off, f[i]);
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+#pragma unroll
+        for (int q = 0; q < NP; ++q) {
+            // (a column of the four-pixel class may end before its third and fourth: whatever
+            // they hold must not reach it)
+            if (NP < 4 || q < 2) run = fmaf(w[q], f[i][q], run);
+            else run += mul_or_zero(w[q], f[i][q]);
+        }
+        lds_store(mine, (unsigned)(k0 + i + 1) * (kWave * 4u), run);
+    }
+}
+
+// First step on one line: ns slices (an even number).
+template <int NP, int K = 0>
+__device__ inline void col_slices_in(const char *line, unsigned off, int64_t plane, int ns, const float *w, char *mine,
+                                     float run)
+{
+    if constexpr (K < kColMax) {
+        if (ns < K + 4) {
+            if (ns > K) col_slices<NP, 2>(line, off, plane, w, K, mine, run);
+            return;
+        }
+        col_slices<NP, 4>(line, off, plane, w, K, mine, run);
+        col_slices_in<NP, K + 4>(line, off, plane, ns, w, mine, run);
+    }
+}
+
+// The same for a column over any number of pixels.
+template <class W>
+__device__ inline void col_slices_any(const char *line, unsigned off, int64_t plane, int ns, int m0, float t1, W weight,
+                                      char *mine)
+{
+    float run = 0.0f;
+    lds_store(mine, 0, 0.0f);
+    for (int k = 0; k < ns; ++k) {
+        for (int m = m0; (float)m < t1; ++m) {
+            float f[1];
+            load_floats<1>(line + k * plane, off + (unsigned)(m - m0) * 4u, f);
+            run = fmaf(weight(m), f[0], run);
+        }
+        lds_store(mine, (unsigned)(k + 1) * (kWave * 4u), run);
+    }
+}
+
+// One detector cell, scaled as cell_store scales it.
+template <int OPK, int GEO>
+__device__ inline void col_store(const ColArgs &a, const ViewHdr &h, const float4 &cc, float d0, float d1,
+                                 float *__restrict__ out, int c, int r, int v, int b, float sum)
+{
+    float s = h.colw;
+    if (OPK == CELL_A) {
+        s = h.delta * cc.z / cc.w;
+        if (GEO != GEO_PAR) {
+            const float dbp = 0.5f * (d0 + d1) - h.P;
+            const float hb = cc.y * (a.v0 + ((float)r + 0.5f) * a.dvv);
+            s /= fabsf(h.S) / sqrtf(dbp * dbp + hb * hb + h.S * h.S);
+        }
+    }
+    out[(((int64_t)b * a.nview + v) * a.nv + r) * a.nu + (h.keep ? c : a.nu - 1 - c)] = sum * s;
+}
+
+// Workgroup bid of the gather (lds: col_lds_bytes).
+template <int OPK, int GEO, bool SPLIT>
+__device__ inline void col_gather(const ColArgs &a, int bid, const float *__restrict__ TX, const float *__restrict__ TY,
+                                  float *__restrict__ out, float *lds)
+{
+    const int lane = threadIdx.x & (kWave - 1), wave = SPLIT ? wave_uniform(threadIdx.x / kWave) : 0;
+    // Row tiles outermost, so that the slices in use at one time are few, and each of the 8
+    // XCDs (workgroups go to them in turn) on a run of neighbouring groups and views, which
+    // read the same pixels: 512^2 x 256 on 736 x 128, 1152 views takes 22.8 ms so, 24.1 without
+    // the runs, 33.1 with row tiles innermost.
+    const int nblk = a.nitems * a.ntile * a.nb, run = nblk >> 3;
+    if (bid < run * 8) bid = (bid & 7) * run + (bid >> 3);
+    const int idx = bid % a.nitems, rt = bid / a.nitems % a.ntile, b = bid / a.nitems / a.ntile;
+    const int item = wave_uniform(ro_load(a.citems + idx));
+    const int v = item / a.ncg, c = (item - v * a.ncg) * kWave + lane;
+    const ViewHdr h = ro_load(a.hdr + v);
+    const CellGroup cg = ro_load(a.cgrp + item);
+    const int r0 = rt * a.rows, nrow = imin(a.rows, a.nv - r0);
+    const float4 *ct = a.col + (int64_t)v * (a.nu + 1) + imin(c, a.nu - 1);
+    const float4 cc = g_load(ct);
+    const float d0 = cc.x, d1 = g_load(&ct[1].x);
+    const float cyv = cc.y * a.vc, cyd = cc.y * a.dvv;
+    const int nline = wave_uniform(h.nline), nal = wave_uniform(h.nalong);
+    const float fal = (float)nal, fnz = (float)a.nz;
+    const int64_t pitch = (int64_t)(nal + kColPad) * 4, plane = pitch * nline;
+    const unsigned plane4 = (unsigned)plane;
+    const char *T = reinterpret_cast<const char *>(wave_uniform(h.xdrv) ? TX : TY) + (int64_t)b * a.nzp * plane;
+    const float4 *lt = a.lineC + (int64_t)v * a.maxline;
+    char *mine = reinterpret_cast<char *>(lds) + (size_t)wave * (a.ns + 1) * (kWave * 4) + lane * 4;
+    const float rf = (float)r0 - 0.5f * (float)a.nv;  // first row boundary from the detector's middle
+    const unsigned mine4 = lds_address(mine);  // (the block of a one-wave workgroup starts at 0)
+    unsigned addr[5] = {mine4, mine4, mine4, mine4, mine4};
+    float acc[kColRows];
+#pragma unroll
+    for (int q = 0; q < kColRows; ++q) acc[q] = 0.0f;
+    const int per = SPLIT ? ceil_div(nline, kWavesPerBlock) : nline;
+    const int L0 = SPLIT ? wave * per : 0, L1 = imin(nline, L0 + per);
+    for (int base = L0; base < L1; base += kWave) {
+        // lane l: the slices of line base + l, and whether its rows may leave the volume
+        int lns;
+        unsigned long long edge, wide[3];
+        {
+            const float4 lc = g_load(lt + imin(base + lane, L1 - 1));
+            const float lz = lc.z, s = cg.wmax * lc.y;  // s: the group's widest column in pixels
+            wide[0] = __builtin_amdgcn_ballot_w64(!(s < 0.99f));
+            wide[1] = __builtin_amdgcn_ballot_w64(!(s < 1.99f));
+            wide[2] = __builtin_amdgcn_ballot_w64(!(s < 2.99f));
+            lns = imin(col_line_slices(cg.sig_hi * a.dvv * lz, a.rows, a.nzp), a.ns);
+            const float h0 = fmaf((float)r0, a.dvv, a.v0), h1 = fmaf((float)(r0 + a.rows), a.dvv, a.v0);
+            const float s0 = cg.sig_lo * lz, s1 = cg.sig_hi * lz;
+            const float lo = fminf(s0 * h0, s1 * h0) + a.zoff, hi = fmaxf(s0 * h1, s1 * h1) + a.zoff;
+            const float tol = fmaf(1e-4f, fmaxf(fabsf(lo), fabsf(hi)) + fabsf(a.zoff), 0.01f);
+            edge = __builtin_amdgcn_ballot_w64(!(lo > tol && hi < fnz - tol));
+        }
+        const int n = imin(kWave, L1 - base);
+        for (int l = 0; l < n; ++l) {
+            const int L = base + l;
+            const float4 lc = ro_load(lt + L);
+            const float t0 = fmaf(d0, lc.y, lc.x), t1 = fmaf(d1, lc.y, lc.x);
+            if (!(t1 > 0.0f && t0 < fal)) continue;
+            const int ns = __builtin_amdgcn_readlane(lns, l);
+            const float dz = cyd * lc.z, z0 = fmaf(cyv, lc.z, a.zoff);
+            const float e0 = maxf_finite(t0, 0.0f), e1 = minf_finite(t1, fal);
+            const int m0 = (int)e0;
+            const float mf = (float)m0;
+            // the lane's slices: from the one its first boundary lies in, inside the tables
+            const int kb = imin(imax((int)fmaf(rf, dz, z0), 0), a.nzp - ns);
+            const float kbf = (float)kb, zr = fmaf(rf, dz, z0 - kbf);
+            const unsigned off = mad24_uniform((unsigned)kb, plane4, (unsigned)m0 * 4u);
+            const char *line = T + L * pitch;
+            auto weight = [&](float ou, int m) -> float {
+                if (OPK == CELL_A) return ou * lc.w;
+                if (OPK == CELL_BWT) {
+                    const float px = h.xdrv ? ((float)m - 0.5f * a.nx + 0.5f) * a.dx + a.shx
+                                            : ((float)L - 0.5f * a.nx + 0.5f) * a.dx + a.shx;
+                    const float py = h.xdrv ? (0.5f * a.ny - (float)L - 0.5f) * a.dy + a.shy
+                                            : ((float)m - 0.5f * a.ny + 0.5f) * a.dy + a.shy;
+                    return ou * fdk_weight<GEO>(h.sx, h.sy, px, py, a.sod);
+                }
+                return ou;
+            };
+            // weights of NP pixels: ends of the overlaps, clipped to the line's end (the
+            // entries past it are zeros)
+            auto fixed = [&](auto np) {
+                constexpr int NP = decltype(np)::value;
+                float w[NP], e = e0;
+#pragma unroll
+                for (int q = 0; q < NP; ++q) {
+                    const float x = q + 1 < NP ? minf_finite(e1, mf + (float)(q + 1)) : e1;
+                    w[q] = weight(x - e, m0 + q);
+                    e = x;
+                }
+                lds_store(mine, 0, 0.0f);
+                col_slices_in<NP>(line, off, plane, ns, w, mine, 0.0f);
+            };
+            if (!(wide[0] >> l & 1)) fixed(std::integral_constant<int, 2>{});
+            else if (!(wide[1] >> l & 1)) fixed(std::integral_constant<int, 3>{});
+            else if (!(wide[2] >> l & 1)) fixed(std::integral_constant<int, 4>{});
+            else
+                col_slices_any(line, off, plane, ns, m0, e1,
+                               [&](int m) { return weight(fminf(e1, (float)(m + 1)) - fmaxf(e0, (float)m), m); }, mine);
+            // second step: row boundaries in slices from the lane's first
+            auto rows = [&](auto clip) {
+                constexpr bool CLIP = decltype(clip)::value;
+                const float zlo = -kbf, zhi = fnz - kbf;
+                auto at = [&](float z, unsigned &ad, float &lo, float &hi) -> float {
+                    if (CLIP) z = clampf(z, zlo, zhi);
+                    if (SPLIT) {
+                        lds_entries(((unsigned)(int)z << 8) + mine4, lo, hi);
+                    } else {
+                        entry_address(ad, z);
+                        lds_entries(ad, lo, hi);
+                    }
+                    return __builtin_amdgcn_fractf(z);
+                };
+                // (the first may round to just below its slice)
+                float lo, hi, fr = at(maxf_finite(zr, 0.0f), addr[4], lo, hi);
+                float Kp = fmaf(fr, hi - lo, lo);
+#pragma unroll
+                for (int g = 0; g < kColRows / 4; ++g) {
+                    if (g * 4 >= nrow) break;
+                    float f[4], e0[4], e1[4];
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) f[i] = at(fmaf((float)(g * 4 + i + 1), dz, zr), addr[i], e0[i], e1[i]);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const float K = fmaf(f[i], e1[i] - e0[i], e0[i]);
+                        acc[g * 4 + i] += K - Kp;
+                        Kp = K;
+                    }
+                }
+            };
+            if (edge >> l & 1) rows(std::true_type{});
+            else rows(std::false_type{});
+        }
+    }
+    if (SPLIT) {  // the quarters' sums in wave order
+        float *part = lds;
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < kColRows; ++q) part[(wave * kColRows + q) * kWave + lane] = acc[q];
+        __syncthreads();
+        if (c >= a.nu) return;
+        for (int q = wave; q < nrow; q += kWavesPerBlock) {
+            float s = part[q * kWave + lane];
+#pragma unroll
+            for (int k = 1; k < kWavesPerBlock; ++k) s += part[(k * kColRows + q) * kWave + lane];
+            col_store<OPK, GEO>(a, h, cc, d0, d1, out, c, r0 + q, v, b, s);
+        }
+        return;
+    }
+    if (c >= a.nu) return;
+#pragma unroll
+    for (int q = 0; q < kColRows; ++q)
+        if (q < nrow) col_store<OPK, GEO>(a, h, cc, d0, d1, out, c, r0 + q, v, b, acc[q]);
+}
+
+#endif
+
+}  // namespace xr

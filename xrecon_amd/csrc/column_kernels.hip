@@ -1,0 +1,161 @@
+// Kernels and launches of the two-step cell gathers (column.h), for one plan and for batches.
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <cstdint>
+
+#include "column.h"
+
+namespace xr {
+
+namespace {
+
+struct ColOne {
+    ColArgs a;
+    const float *in;
+    float *out, *t0, *t1;
+};
+
+// Instances of a batch; those that another launch covers count no blocks.
+struct ColMany {
+    const ColArgs *args;  // device array
+    int n;
+    ColLaunch l;
+};
+
+struct ColJob {
+    ColArgs a;
+    const float *in;
+    float *out, *t0, *t1;
+    int bid;
+};
+
+__device__ inline bool col_job(const ColOne &o, ColJob &j)
+{
+    j.a = o.a; j.in = o.in; j.out = o.out; j.t0 = o.t0; j.t1 = o.t1;
+    j.bid = blockIdx.x;
+    return true;
+}
+__device__ inline bool col_job(const ColMany &m, ColJob &j)
+{
+    const int bid = blockIdx.x;
+    int i = 0;
+    while (i + 1 < m.n && bid >= m.l.start[i + 1]) ++i;
+    if (bid >= m.l.start[m.n]) return false;
+    j.a = ro_load(m.args + i);
+    j.in = m.l.in[i]; j.out = m.l.out[i]; j.t0 = m.l.t0[i]; j.t1 = m.l.t1[i];
+    j.bid = bid - m.l.start[i];
+    return true;
+}
+
+template <class SRC>
+__global__ __launch_bounds__(kBlock) void k_col_tables(SRC src)
+{
+    ColJob j;
+    if (col_job(src, j)) col_tables(j.a, j.bid, j.in, j.t0, j.t1);
+}
+template <int OPK, int GEO, bool SPLIT, class SRC>
+__global__ __launch_bounds__(SPLIT ? kBlock : kWave) __attribute__((amdgpu_waves_per_eu(5))) void k_col_gather(SRC src)
+{
+    extern __shared__ float col_lds[];
+    ColJob j;
+    if (col_job(src, j)) col_gather<OPK, GEO, SPLIT>(j.a, j.bid, j.t0, j.t1, j.out, col_lds);
+}
+
+template <int OPK, int GEO, class SRC>
+void launch_gather(bool split, unsigned grid, size_t lds, const SRC &src, hipStream_t s)
+{
+    if (split) hipLaunchKernelGGL((k_col_gather<OPK, GEO, true, SRC>), dim3(grid), dim3(kBlock), lds, s, src);
+    else hipLaunchKernelGGL((k_col_gather<OPK, GEO, false, SRC>), dim3(grid), dim3(kWave), lds, s, src);
+}
+
+template <class SRC>
+void launch_any(ColPass pass, int kind, int kop, bool split, unsigned grid, size_t lds, const SRC &src, hipStream_t s)
+{
+    if (pass == COL_TABLES) {
+        hipLaunchKernelGGL((k_col_tables<SRC>), dim3(grid), dim3(kBlock), 0, s, src);
+        return;
+    }
+    // A's cells only tell parallel beams from the others, B^T's are alike
+    if (kop == CELL_A) {
+        if (kind == GEO_PAR) launch_gather<CELL_A, GEO_PAR>(split, grid, lds, src, s);
+        else launch_gather<CELL_A, GEO_FLAT>(split, grid, lds, src, s);
+    } else if (kop == CELL_BT) {
+        launch_gather<CELL_BT, GEO_FLAT>(split, grid, lds, src, s);
+    } else if (kind == GEO_FLAT) {
+        launch_gather<CELL_BWT, GEO_FLAT>(split, grid, lds, src, s);
+    } else if (kind == GEO_ARC) {
+        launch_gather<CELL_BWT, GEO_ARC>(split, grid, lds, src, s);
+    } else {
+        launch_gather<CELL_BWT, GEO_PAR>(split, grid, lds, src, s);
+    }
+}
+
+}  // namespace
+
+int64_t col_pass_blocks(ColPass pass, const ColArgs &a) { return pass == COL_TABLES ? col_table_blocks(a) : col_blocks(a); }
+
+float *col_second_table(const Plan3d &p, void *ws, int nb)
+{
+    return reinterpret_cast<float *>(static_cast<char *>(ws) + align256((size_t)col_table_floats(p, nb, false) * sizeof(float)));
+}
+
+int col_run(const Plan3d &p, ColPass pass, int kop, const float *in, float *out, int nb, void *ws, hipStream_t s)
+{
+    ColOne o;
+    o.a = make_col_args(p, nb);
+    o.in = in;
+    o.out = out;
+    o.t0 = static_cast<float *>(ws);
+    o.t1 = col_second_table(p, ws, nb);
+    const int64_t grid = col_pass_blocks(pass, o.a);
+    if (grid >= ((int64_t)1 << 31)) return fail(XR_EINVAL, "batch too large for one launch of the cell gather");
+    launch_any(pass, p.kind, kop, o.a.split, (unsigned)grid, col_lds_bytes(o.a), o, s);
+    return XR_OK;
+}
+
+void col_run_many(ColPass pass, int kind, int kop, bool split, size_t lds, const ColArgs *args, int n,
+                  const ColLaunch &l, hipStream_t s)
+{
+    ColMany m;
+    m.args = args;
+    m.n = n;
+    m.l = l;
+    launch_any(pass, kind, kop, split, (unsigned)l.start[n], lds, m, s);
+}
+
+// Rows per tile, LDS slices and line splitting of the two-step gather (Plan3d::col_*).
+void column_plan(Plan3d &p, const PlanTables &t)
+{
+    p.col_rows = p.col_ns = p.col_split = 0;
+    const int nx = p.vol.nx, ny = p.vol.ny, nv = p.geo.nv, nzp = col_slices(p.vol.nz);
+    const int64_t px = (int64_t)(nx + kColPad) * ny * 4, py = (int64_t)(ny + kColPad) * nx * 4;
+    const int64_t plane = px > py ? px : py;
+    if (p.big || p.nview == 0 || plane >= (1 << 24) || plane * nzp >= ((int64_t)1 << 32)) return;
+    const int ncg = ceil_div(p.geo.nu, kWave);
+    float step = 0.0f;  // tallest row of a column on a line that it meets, in slices
+    for (int v = 0; v < p.nview; ++v) {
+        const float4 *lc = t.lineC.data() + (size_t)v * p.maxline, *col = t.col.data() + (size_t)v * (p.geo.nu + 1);
+        for (int g = 0; g < ncg; ++g) {
+            const float sg = t.cgrp[(size_t)v * ncg + g].sig_hi * p.dvv;
+            const float d0 = col[g * kWave].x, d1 = col[imin((g + 1) * kWave, p.geo.nu)].x;
+            for (int L = 0; L < t.hdr[v].nline; ++L) {
+                if (sg * lc[L].z <= step) continue;
+                // (a pixel of slack: the kernel's test is the same up to rounding)
+                const float t0 = fmaf(d0, lc[L].y, lc[L].x), t1 = fmaf(d1, lc[L].y, lc[L].x);
+                if (t1 > -1.0f && t0 < (float)(t.hdr[v].nalong + 1)) step = sg * lc[L].z;
+            }
+        }
+    }
+    if (!(step < 1e4f)) return;
+    for (int rows = kColRows; rows >= 4; rows -= 4) {
+        const int ns = col_line_slices(step, rows, nzp);
+        if (ns > (rows > 4 ? kColFit : kColMax)) continue;
+        p.col_rows = (ceil_div(nv, ceil_div(nv, rows)) + 3) / 4 * 4;  // even tiles
+        p.col_ns = col_line_slices(step, p.col_rows, nzp);
+        p.col_split = (int64_t)p.nview * ncg * ceil_div(nv, p.col_rows) < kColSplitMax ? 1 : 0;
+        return;
+    }
+}
+
+}  // namespace xr

@@ -418,6 +418,18 @@ __host__ __device__ inline void fmac(float &acc, float a, float b)
 #endif
 }
 
+// w x, zero where w is zero, whatever x holds: one v_mul_legacy_f32.
+__host__ __device__ inline float mul_or_zero(float w, float x)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    float r;
+    asm("v_mul_legacy_f32 %0, %1, %2" : "=v"(r) : "v"(w), "v"(x));
+    return r;
+#else
+    return w == 0.0f ? 0.0f : w * x;
+#endif
+}
+
 // A uniform value the compiler takes as new at this place, so that it does not keep
 // results derived from it (a scalar register pair per branch condition) across a loop.
 __host__ __device__ inline unsigned fresh(unsigned x)

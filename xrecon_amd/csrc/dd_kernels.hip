@@ -37,6 +37,7 @@
 #include <algorithm>
 #include <cstdint>
 
+#include "column.h"
 #include "slice.h"
 
 namespace xr {
@@ -631,7 +632,9 @@ size_t workspace_bytes(const Plan3d &p, int op, int nbatch)
     if (rt.kop < 0) return 0;
     if (is_slice(p))
         return slice_table_bytes(p, rt.cell, nbatch) + (op == XR_OP_BACKPROJECTION_W ? align256(fdk_taps_bytes(p)) : 0);
-    if (rt.cell) return align256(vol_prefix_bytes(p, nbatch)) * (p.any_y ? 2 : 1);
+    // (one size whichever cell gather the plan takes)
+    if (rt.cell)
+        return std::max(align256(vol_prefix_bytes(p, nbatch)) * (p.any_y ? 2 : 1), col_table_bytes(p, nbatch));
     size_t tail = split_partial_bytes(p, nbatch);
     if (op == XR_OP_BACKPROJECTION_W) tail = std::max(tail, fdk_taps_bytes(p));  // FDK filter taps
     return align256(sino_prefix_bytes(p, nbatch)) + align256(tail);
@@ -688,7 +691,13 @@ int execute_phase(const Plan3d &p, int op, int phase, const float *in, float *ou
                        ((int64_t)1 << 31))
         return fail(XR_EINVAL, "batch too large for one launch of the cell gather (column groups / 4 x rows x batch "
                                "must stay below 2^31)");
-    if (rt.cell) {
+    if (rt.cell && p.col_rows > 0) {
+        // (tile_rows has nothing to choose here)
+        int rc = XR_OK;
+        if (do_prefix) rc = col_run(p, COL_TABLES, rt.kop, in, nullptr, nbatch, ws, s);
+        if (!rc && do_gather) rc = col_run(p, COL_GATHER, rt.kop, nullptr, out, nbatch, ws, s);
+        if (rc) return rc;
+    } else if (rt.cell) {
         float2 *WX = static_cast<float2 *>(ws);
         float2 *WY = p.any_y ? reinterpret_cast<float2 *>(static_cast<char *>(ws) + align256(vol_prefix_bytes(p, nbatch)))
                              : nullptr;

@@ -116,18 +116,6 @@ void slice_run_many(SlicePass pass, int kind, int kop, int bg, int waves, const 
 
 #if defined(__HIPCC__)
 
-// w x, zero where w is zero, whatever x holds: one v_mul_legacy_f32.
-__device__ inline float mul_or_zero(float w, float x)
-{
-#if defined(__HIP_DEVICE_COMPILE__)
-    float r;
-    asm("v_mul_legacy_f32 %0, %1, %2" : "=v"(r) : "v"(w), "v"(x));
-    return r;
-#else
-    return w == 0.0f ? 0.0f : w * x;
-#endif
-}
-
 // Copies of the images in both line orientations: TX[g][j][m = i][b] and
 // TY[g][i][m = Ny-1-j][b], zeros after each line (32 x 32 tiles, transposed through LDS).
 template <int BG>

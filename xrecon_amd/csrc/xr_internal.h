@@ -95,6 +95,9 @@ struct Plan3d {
     int any_x = 0, any_y = 0;
     int big = 0;             // z-prefix table of one batch item >= 2^32 bytes or plane >= 2^24 bytes
     int vox_fit = 0;         // vox_fit_bit(KC, NI) set: every block of the voxel gather fits the LDS then
+    int col_rows = 0;        // two-step cell gather (column.h): rows per tile, 0: the plan does not take it
+    int col_ns = 0;          // ... LDS slices per lane
+    int col_split = 0;       // ... 1: the waves of a workgroup share one item's lines
     int vsplit = 1;          // voxel gathers: views split over this many workgroup sets (summed after)
     // Scalars shared by all views.
     float zb = 0, dz = 1;    // volume bottom z and slice thickness
