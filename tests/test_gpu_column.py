@@ -22,7 +22,7 @@ SIZES = {
     "one_tile": (24, 20, 17, 64, 16, 1.0, 0.5, 0.9, 0.0, 0.0, 40),
     "tile_and_row": (33, 19, 37, 65, 17, 1.1, 0.7, 0.9, 0.3, -0.4, 40),
     "off_volume": (30, 40, 20, 70, 45, 1.0, 0.7, 0.9, -6.0, 3.0, 40),  # rows above and below the volume
-    "unsplit": (24, 20, 9, 130, 40, 1.0, 0.4, 0.5, 0.0, 0.1, 1200),  # more waves than line quarters need
+    "unsplit": (24, 20, 9, 129, 33, 1.0, 0.4, 0.5, 0.0, 0.1, 3700),  # more waves than line quarters need
     "tall_rows": (25, 31, 61, 40, 11, 0.5, 0.9, 1.7, 0.2, 0.3, 40),  # tiles of 4 and 8 rows
     "taller_rows": (20, 20, 90, 40, 7, 0.25, 0.9, 2.9, 0.0, 0.0, 40),  # beyond 9 slices per row
     "four_pixels": (50, 50, 12, 21, 10, 1.0, 1.9, 1.0, 0.0, 0.0, 40),

@@ -20,7 +20,7 @@
 // (Plan3d::col_rows > 0) when its tiles' slices fit the LDS (column_plan).  The z-prefix
 // gathers remain for rows of more than 9 slices and for volumes beyond 24-bit planes or
 // 32-bit offsets.  Whole call before and after: 256^2 x 64, 720 views of 512 x 64 flat 2.84
-// and 2.00 ms; 256^2 x 10, 360 views of 256 x 10 0.34 and 0.23 ms; 512^2 x 256, 1152 views of
+// and 1.85 ms; 256^2 x 10, 360 views of 256 x 10 0.34 and 0.15 ms; 512^2 x 256, 1152 views of
 // 736 x 128 arc 30.6 and 20.1 ms.
 #pragma once
 
@@ -37,10 +37,12 @@ constexpr int kColRows = 16;    // most rows of a tile
 // the registers allow.  512^2 x 256 on 736 x 128, 1152 views: 16 rows with 36 slices 24.1 ms,
 // 8 rows with 20 slices 25.5 ms (4 rows 44.5 ms with 12), 16 rows with 22 slices 19.7 ms.
 constexpr int kColFit = 30;
-// Fewer waves than this (an MI355X holds 5120) split their lines over four: 1440 waves
-// (256^2 x 10, 360 views) take 0.24 ms split and 0.42 unsplit, 7218 take 1.14 and 1.13, 8640
-// 1.16 and 1.19, 23040 2.14 and 2.13.
-constexpr int64_t kColSplitMax = 8192;
+// Fewer waves than this split their lines over the four waves of a workgroup.  The split form
+// runs 6 waves per SIMD (a few registers spill, and few waves finish evenly), the other 5:
+// 1440 waves (256^2 x 10, 360 views) take 0.17 ms split and 0.45 unsplit, 7218 1.05 and 1.12,
+// 8640 1.10 and 1.12, 23040 (256^2 x 64, 720 views) 2.00 and 2.10, 110592 (512^2 x 256) 21.9
+// and 19.7.  With 5 waves the first takes 0.24: its 5760 quarters are then just over one round.
+constexpr int64_t kColSplitMax = 32768;
 
 struct ColArgs {
     const ViewHdr *hdr;

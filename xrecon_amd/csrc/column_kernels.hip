@@ -55,7 +55,7 @@ __global__ __launch_bounds__(kBlock) void k_col_tables(SRC src)
     if (col_job(src, j)) col_tables(j.a, j.bid, j.in, j.t0, j.t1);
 }
 template <int OPK, int GEO, bool SPLIT, class SRC>
-__global__ __launch_bounds__(SPLIT ? kBlock : kWave) __attribute__((amdgpu_waves_per_eu(5))) void k_col_gather(SRC src)
+__global__ __launch_bounds__(SPLIT ? kBlock : kWave) __attribute__((amdgpu_waves_per_eu(SPLIT ? 6 : 5))) void k_col_gather(SRC src)
 {
     extern __shared__ float col_lds[];
     ColJob j;
@@ -131,19 +131,23 @@ void column_plan(Plan3d &p, const PlanTables &t)
     const int nx = p.vol.nx, ny = p.vol.ny, nv = p.geo.nv, nzp = col_slices(p.vol.nz);
     const int64_t px = (int64_t)(nx + kColPad) * ny * 4, py = (int64_t)(ny + kColPad) * nx * 4;
     const int64_t plane = px > py ? px : py;
-    if (p.big || p.nview == 0 || plane >= (1 << 24) || plane * nzp >= ((int64_t)1 << 32)) return;
+    if (p.is2d || p.big || p.nview == 0 || plane >= (1 << 24) || plane * nzp >= ((int64_t)1 << 32)) return;
     const int ncg = ceil_div(p.geo.nu, kWave);
     float step = 0.0f;  // tallest row of a column on a line that it meets, in slices
     for (int v = 0; v < p.nview; ++v) {
-        const float4 *lc = t.lineC.data() + (size_t)v * p.maxline, *col = t.col.data() + (size_t)v * (p.geo.nu + 1);
+        const float4 *lines = t.lineC.data() + (size_t)v * p.maxline;
+        float top = 0.0f;  // (most groups need no walk over the lines)
+        for (int L = 0; L < t.hdr[v].nline; ++L) top = std::max(top, lines[L].z);
+        const float4 *col = t.col.data() + (size_t)v * (p.geo.nu + 1);
         for (int g = 0; g < ncg; ++g) {
             const float sg = t.cgrp[(size_t)v * ncg + g].sig_hi * p.dvv;
+            if (sg * top <= step) continue;
             const float d0 = col[g * kWave].x, d1 = col[imin((g + 1) * kWave, p.geo.nu)].x;
             for (int L = 0; L < t.hdr[v].nline; ++L) {
-                if (sg * lc[L].z <= step) continue;
+                if (sg * lines[L].z <= step) continue;
                 // (a pixel of slack: the kernel's test is the same up to rounding)
-                const float t0 = fmaf(d0, lc[L].y, lc[L].x), t1 = fmaf(d1, lc[L].y, lc[L].x);
-                if (t1 > -1.0f && t0 < (float)(t.hdr[v].nalong + 1)) step = sg * lc[L].z;
+                const float t0 = fmaf(d0, lines[L].y, lines[L].x), t1 = fmaf(d1, lines[L].y, lines[L].x);
+                if (t1 > -1.0f && t0 < (float)(t.hdr[v].nalong + 1)) step = sg * lines[L].z;
             }
         }
     }

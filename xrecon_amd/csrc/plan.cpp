@@ -396,8 +396,9 @@ int build_tables(Plan3d &p, const float *angles, PlanTables &t, std::string &err
             }
     }
     const VoxArgs va = make_vox_args(p, 1, 1);
-    int misses = 0;
+    int misses = is2d ? 31 : 0;  // (2D: slice.h)
     for (const VoxTile &vt : t.vtile) {
+        if (misses == 31) break;
         if (!(misses & 1) && !voxel_tile_fits<8, 1>(vt, va)) misses |= vox_fit_bit(8, 1);
         if (!(misses & 2) && !voxel_tile_fits<16, 1>(vt, va)) misses |= vox_fit_bit(16, 1);
         if (!(misses & 4) && !voxel_tile_fits<32, 1>(vt, va)) misses |= vox_fit_bit(32, 1);
