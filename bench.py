@@ -290,7 +290,7 @@ def bench_cfg5(dev, reps):
                        "1152 views, B=4, 32 random ellipsoids each (intensities 0-0.05/mm, seeds 1005-1008)",
            "voxel_views_per_operator": vv, "value": vv / ((t_a + t_b) * 1e-3), "unit": "voxel-views/s",
            "ms_A": t_a, "ms_B": t_b, "ms_AT": t_at, "adjoint_value": vv / ((t_a + t_at) * 1e-3),
-           "tiles": "defaults (8 rows, LDS-staged cell gather; 32 slices in halves of 16)"}
+           "tiles": "defaults (16-row tiles of the two-step cell gather; voxel slices in groups of four)"}
     try:
         nnz = nnz_of(CFG5_WORKLOAD) * NB
     except (KeyError, OSError):
@@ -385,7 +385,8 @@ def bench_cfg5_unrolled(dev, iterations=10):
 # Sources that decide the single-plan gather kernels' code and tables: a traffic figure
 # measured on other sources is reported as not current.
 KERNEL_SOURCES = ("xrecon_amd/csrc/dd_body.h", "xrecon_amd/csrc/dd_kernels.hip", "xrecon_amd/csrc/xr_internal.h",
-                  "xrecon_amd/csrc/plan.cpp")
+                  "xrecon_amd/csrc/plan.cpp", "xrecon_amd/csrc/column.h", "xrecon_amd/csrc/column_kernels.hip",
+                  "xrecon_amd/csrc/slice.h", "xrecon_amd/csrc/slice_kernels.hip")
 
 
 def kernel_sources_digest():
@@ -620,26 +621,13 @@ def main():
     nnz = nnz_of(WORKLOAD)
     flops = 4.0 * nnz
     if t_cell >= t_vox:
-        # one launch per span class of the column groups (two-pixel at the tuned rows,
-        # three-pixel and general at most 8 rows)
-        ncls = plan.cell_classes()
-        r_a = tune_a[0] & 0xFF
-        rows = (r_a, min(r_a, 8), min(r_a, 8))
-        # LDS-staged classes 2 and 3 at 4 rows and more: as tuned (this table is below the
-        # 128 MiB the library stages by default)
-        staged = bool(tune_a[0] & autotune.CELL_LDS)
-        blocks = [-(-n // 4) * -(-wl["Nv"] // r) for r, n in zip(rows, ncls)]
-        if -(-sum(ncls) // 4) * -(-wl["Nv"] // r_a) < 4096:  # small grids: one launch for all classes
-            symbol = [f"k_cell<0, 1, {r_a}, -1, false, false>"]
-        else:  # a class launch stages only with 4096 workgroups or more
-            symbol = [f"k_cell<0, 1, {r}, {span}, false, "
-                      f"{'true' if staged and span and r >= 4 and nb >= 4096 else 'false'}>"
-                      for r, span, n, nb in zip(rows, (2, 3, 0), ncls, blocks) if n > 0]
+        # the two-step gather of flat cones, its lines split over the four waves of a workgroup
+        symbol = "k_col_gather<0, 1, true>"
         dominant, t_dom = "cell_gather(A)", t_cell
     else:
         kc = tune_b[1]
         dominant, t_dom = "voxel_gather(B)", t_vox
-        symbol = f"k_voxel<0, 1, {kc & 0xff}, {'true' if kc & 0x100 else 'false'}>"
+        symbol = f"k_voxel<0, 1, {kc & 0xff}, 1, true>"  # (one item; every block fits the LDS)
     achieved = flops / (t_dom * 1e-3) / 1e12
     traffic, traffic_src = traffic_from_profiles(symbol)
     # the summary's kernels are these only if it was taken on the same kernel sources
