@@ -3,14 +3,16 @@
 Two knobs exist, one per kernel family (``Plan.kernel_kind(op)``):
 
 * cell gathers (A, B^T, B_W^T): ``tile_rows`` in {1, 2, 4, 8, 16} -- detector rows per
-  thread.  More rows amortise each line's column overlaps and share row boundaries,
+  thread -- for the few 3D plans that gather from z-prefix tables (rows of more than 9
+  slices, planes beyond 24-bit offsets); the others choose their tiles themselves and every
+  candidate is the same kernel.  More rows amortise each line's column overlaps and share row boundaries,
   but cost registers and therefore resident waves.  Tiles of 4 rows and more are also
   tried with CELL_LDS and CELL_DIRECT: each workgroup's table lookups served from
   blocks staged in LDS, or read from device memory (the same results either way).
 * voxel gathers (B, B_W, A^T): ``voxel_chunk`` in {1, 4, 8, 16} -- slices per thread --
-  and 16 | VOXEL_HALVES, 32 | VOXEL_HALVES: 16 or 32 slices run as two halves that a wave
-  skips when none of its lanes reaches the detector in them.  Longer chunks amortise each view's column search,
-  shorter ones give more waves; the halves pay on tall volumes.
+  and 16 | VOXEL_HALVES (the same as 16), 32 | VOXEL_HALVES.  A wave skips the groups of 4
+  slices in which none of its lanes reaches the detector.  Longer chunks amortise each
+  view's column search, shorter ones give more waves; 32 slices pay on tall volumes.
 
 ``tune`` times the gather pass alone (the prefix pass is shared) for every candidate
 with HIP events on the caller's stream, takes the median of a few launches, and keeps
